@@ -242,17 +242,36 @@ typedef struct {
 
 int ssa_sparse_gather_attention_bwd(const ssa_apply_bwd_args *a, void *stream);
 
-/* Deterministic backward (the reference's CPU autograd through
- * sparse_attention.py:1146-1199 is deterministic; ssa_sparse_gather_attention_bwd
- * adds dk / dv with fp32 atomics, whose order varies).  Same arguments and
- * results; each key row's terms are rounded to a fixed-point grid of that
- * row (the finest for which slot count x largest weight x largest |q| or
- * |dout| cannot overflow 64 bits) and summed as integers, so every run gives
- * the same bits.  Needs a 256-byte aligned workspace of
- * ssa_sparse_gather_attention_bwd_det_workspace_bytes (8 bytes per slot, 16
- * per key row element and 12 per key row); a key row whose bound is not
- * finite gets NaN.  SparseAttention takes it under
- * torch.use_deterministic_algorithms(True). */
+/* Gradients of ssa_sparse_gather_attention through the transposed graph: every
+ * key row's dk and dv is summed in registers by the wavefronts that own it, so
+ * no memory is added to by atomics (ssa_sparse_gather_attention_bwd does that,
+ * and needs no workspace).
+ *   fwd: the forward's arguments (out is not read or written; neighbors and
+ *   valid, or neighbors32); dout (B,Hq,N,d) in q's type or fp32; dq (B,Hq,N,d),
+ *   dk and dv (B,Hkv,M,d), all in q's type or all fp32, are WRITTEN.  Views with
+ *   a unit last stride.  Sums in fp32, rounded once.
+ *   deterministic: the same bits on every run (fp64 sums of terms rounded to a
+ *   grid of the key row, exact in any order); a key row whose bound (slots x
+ *   largest weight x largest |q| or |dout|) is not finite gets NaN.
+ * Needs a 256-byte aligned workspace of
+ * ssa_sparse_gather_attention_grad_workspace_bytes: about 20 bytes per slot of
+ * as many (batch, kv head) groups as hold 2^28 slots (at least one). */
+typedef struct {
+    ssa_apply_args fwd;
+    ssa_tensor4 dout;
+    ssa_tensor4 dq, dk, dv;
+    int32_t deterministic;
+} ssa_apply_grad_args;
+
+int64_t ssa_sparse_gather_attention_grad_workspace_bytes(const ssa_apply_grad_args *a);
+int ssa_sparse_gather_attention_grad(const ssa_apply_grad_args *a, void *workspace,
+                                     int64_t workspace_bytes, void *stream);
+
+/* Deterministic backward with the arguments and results of
+ * ssa_sparse_gather_attention_bwd (fp32 dout and gradients, dk and dv
+ * ACCUMULATED): the deterministic form of ssa_sparse_gather_attention_grad.
+ * Needs a 256-byte aligned workspace of
+ * ssa_sparse_gather_attention_bwd_det_workspace_bytes. */
 int64_t ssa_sparse_gather_attention_bwd_det_workspace_bytes(const ssa_apply_bwd_args *a);
 int ssa_sparse_gather_attention_bwd_det(const ssa_apply_bwd_args *a, void *workspace,
                                         int64_t workspace_bytes, void *stream);

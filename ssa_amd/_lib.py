@@ -69,6 +69,11 @@ class ApplyBwdArgs(ctypes.Structure):
     _fields_ = [("fwd", ApplyArgs), ("dout", c_vp), ("dq", c_vp), ("dk", c_vp), ("dv", c_vp)]
 
 
+class ApplyGradArgs(ctypes.Structure):
+    _fields_ = [("fwd", ApplyArgs), ("dout", Tensor4), ("dq", Tensor4), ("dk", Tensor4),
+                ("dv", Tensor4), ("deterministic", c_i32)]
+
+
 _lib = None
 _override = None
 CHECKED_LIB_PATH = os.path.join(_HERE, "libssa_amd_checked.so")
@@ -161,6 +166,11 @@ def _configure(L):
     L.ssa_sparse_gather_attention_bwd_det.restype = ctypes.c_int
     L.ssa_sparse_gather_attention_bwd_det.argtypes = [ctypes.POINTER(ApplyBwdArgs), c_vp, c_i64,
                                                       c_vp]
+    L.ssa_sparse_gather_attention_grad_workspace_bytes.restype = c_i64
+    L.ssa_sparse_gather_attention_grad_workspace_bytes.argtypes = [ctypes.POINTER(ApplyGradArgs)]
+    L.ssa_sparse_gather_attention_grad.restype = ctypes.c_int
+    L.ssa_sparse_gather_attention_grad.argtypes = [ctypes.POINTER(ApplyGradArgs), c_vp, c_i64,
+                                                   c_vp]
     L.ssa_checked_oob.restype = ctypes.c_int
     L.ssa_checked_oob.argtypes = [ctypes.POINTER(ctypes.c_uint32)]
     return L
@@ -607,6 +617,46 @@ def gather_attention_bwd(q, k, v, neighbors, valid, scale, fp32w, dropout_p, see
                "sparse_gather_attention_bwd")
     del keep
     return dq, dk, dv
+
+
+def gather_attention_grad(q, k, v, neighbors, valid, scale, fp32w, dropout_p, seed, dout,
+                          deterministic=False):
+    """dq, dk, dv in q's dtype (ssa_sparse_gather_attention_grad: the key rows'
+    gradients summed over the transposed graph; a workspace is allocated
+    here).  deterministic: the same bits on every run."""
+    check_apply_shapes(q, k, v, neighbors, valid, dout)
+    require_device(q, k, v, neighbors, valid, dout)
+    d = q.shape[-1]
+    dp = kernel_head_dim(d, q.dtype)
+    if dp != d:
+        # head dims the kernels do not take: run zero-padded, keep the d columns
+        grads = gather_attention_grad(_pad_cols(q, dp), _pad_cols(k, dp), _pad_cols(v, dp),
+                                      neighbors, valid, scale, fp32w, dropout_p, seed,
+                                      _pad_cols(dout, dp), deterministic)
+        return tuple(t[..., :d].contiguous() for t in grads)
+    if dout.dtype not in (q.dtype, torch.float32):
+        dout = dout.to(torch.float32)
+    # gradients in their operands' memory order (a view over a projection's
+    # output then takes its gradient without another copy)
+    grads = [torch.empty_like(t) for t in (q, k, v)]
+    grads = [t if t.stride(-1) == 1 else torch.empty(t.shape, dtype=t.dtype, device=t.device)
+             for t in grads]
+    f, keep = _apply_args(q, k, v, neighbors, valid, scale, fp32w, dropout_p, seed, grads[0])
+    a = ApplyGradArgs()
+    a.fwd = f
+    a.dout, do = view4(dout)
+    (a.dq, _), (a.dk, _), (a.dv, _) = (view4(t) for t in grads)
+    a.deterministic = int(deterministic)
+    L = lib()
+    wsb = L.ssa_sparse_gather_attention_grad_workspace_bytes(ctypes.byref(a))
+    if wsb < 0:
+        _check(int(wsb), "sparse_gather_attention_grad")
+    ws = torch.empty(max(int(wsb), 1), dtype=torch.uint8, device=q.device)
+    _check(L.ssa_sparse_gather_attention_grad(ctypes.byref(a), ws.data_ptr(), int(wsb),
+                                              _stream(q)), "sparse_gather_attention_grad")
+    # the allocator orders the reuse of these after this stream's work
+    del ws, keep, do
+    return tuple(grads)
 
 
 # --------------------------------------------------------------------------- measurement

@@ -15,133 +15,9 @@
 // !valid; p = exp(s - max) / sum in fp32; 16-bit models round p to the value
 // dtype before P.V (fp32_attn_weights keeps it fp32); P.V accumulates in fp32
 // and is rounded once to the output dtype.
-#include <type_traits>
-
-#include "ssa_common.h"
+#include "ssa_apply_dev.h"
 
 namespace {
-
-struct ApplyP {
-    int32_t B, Hq, Hkv, N, M, K, rep;
-    int32_t d;             // head dim (<= the kernel's D; lanes past it load zeros, store nothing)
-    const void *q, *k, *v;
-    int64_t qsb, qsh, qsn, ksb, ksh, ksn, vsb, vsh, vsn;
-    const int64_t *nb;
-    const uint8_t *valid;
-    const int32_t *nb32;   // or the graph as int32 ids, negative = invalid
-    int32_t *row_inv;      // optional: per row, its count of invalid slots
-    float scale;
-    int32_t fp32w;
-    float drop_p;
-    float drop_scale;
-    uint64_t seed;
-    void *out;
-    int64_t osb, osh, osn;
-    int64_t rows;          // B*Hq*N
-    int64_t nblocks;       // logical blocks
-    // backward
-    const float *dout;
-    float *dq, *dk, *dv;
-    // deterministic backward (workspace): per (row, slot) the two weights the
-    // key and value gradients take, per key row its slot count and largest
-    // weights (float bits), the largest |q| and |dout| (float bits), and the
-    // fixed-point sums
-    float *wdraw, *wpw;
-    uint32_t *kcnt, *kmaxd, *kmaxp, *gmax;
-    unsigned long long *acck, *accv;
-};
-
-constexpr int WAVES = 4;   // waves per workgroup
-
-template <typename T> struct VecOf;
-template <> struct VecOf<float> { static constexpr int n = 4; };
-template <> struct VecOf<bf16_t> { static constexpr int n = 8; };
-template <> struct VecOf<f16_t> { static constexpr int n = 8; };
-
-template <typename T, int D> struct Geo {
-    // elements per lane: a 16-byte load, more when the row is wider than a
-    // wave holds that way (fp32 beyond 256)
-    static constexpr int VEC = (VecOf<T>::n < D) ? (VecOf<T>::n * SSA_WAVE < D ? D / SSA_WAVE
-                                                                              : VecOf<T>::n)
-                                                 : D;
-    static constexpr int LPR = D / VEC;                                // lanes per row
-    static constexpr int RPI = SSA_WAVE / LPR;                         // rows per wave load
-    static_assert(D % VEC == 0, "head dim must be a multiple of the vector width");
-    static_assert(LPR <= SSA_WAVE, "row wider than a wave");
-};
-
-template <typename T, int VEC>
-__device__ __forceinline__ void load_vec(const T *p, float (&f)[VEC]) {
-    if constexpr (sizeof(T) * VEC == 32) {
-        uint4 u[2] = {reinterpret_cast<const uint4 *>(p)[0], reinterpret_cast<const uint4 *>(p)[1]};
-        const T *e = reinterpret_cast<const T *>(u);
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) f[i] = to_f32(e[i]);
-    } else if constexpr (sizeof(T) * VEC == 16) {
-        uint4 u = *reinterpret_cast<const uint4 *>(p);
-        const T *e = reinterpret_cast<const T *>(&u);
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) f[i] = to_f32(e[i]);
-    } else if constexpr (sizeof(T) * VEC == 8) {
-        uint2 u = *reinterpret_cast<const uint2 *>(p);
-        const T *e = reinterpret_cast<const T *>(&u);
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) f[i] = to_f32(e[i]);
-    } else {
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) f[i] = to_f32(p[i]);
-    }
-}
-
-// counter-based uniform in [0, 1): 64-bit mix of (seed, row, slot)
-__device__ __forceinline__ float drop_uniform(uint64_t seed, int64_t row, int j) {
-    uint64_t x = seed ^ (uint64_t)row * 0x9E3779B97F4A7C15ull ^ ((uint64_t)j << 32);
-    x ^= x >> 33; x *= 0xff51afd7ed558ccdull;
-    x ^= x >> 33; x *= 0xc4ceb9fe1a85ec53ull;
-    x ^= x >> 33;
-    return (float)(x >> 40) * (1.0f / 16777216.0f);
-}
-
-// The factor kept weights are multiplied by: the reference's dropout runs on
-// the weights in their own dtype (the value dtype, or fp32 with
-// fp32_attn_weights), whose noise tensor holds 1 / (1 - p) rounded to that
-// dtype (sparse_attention.py:1193-1194).
-template <typename T>
-__device__ __forceinline__ float drop_scale_of(const ApplyP &p) {
-    return p.fp32w ? p.drop_scale : Cvt<T>::round(p.drop_scale);
-}
-
-// A query row's graph slots j0 + u * 64 + lane (u < NB): the ids (int32 graph,
-// or int64 ids and the mask) of all NB groups are loaded before any is used,
-// so the row pays one memory latency for them instead of one per group.  The
-// loads are unconditional (lanes past the row read its last slot) and the
-// graph's layout is a template parameter, so no branch separates a load from
-// the others.
-constexpr int APPLY_SLOT_BATCH = 4;
-template <int NB, bool I32>
-struct RowSlots {
-    int64_t y[NB];
-    uint8_t v[NB];
-    __device__ __forceinline__ void load(const ApplyP &p, int64_t row, const int64_t *nb,
-                                         const uint8_t *va, int j0, int lane) {
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-            const int j = min(j0 + u * SSA_WAVE + lane, p.K - 1);
-            if constexpr (I32) {
-                y[u] = p.nb32[row * p.K + j];
-            } else {
-                y[u] = nb[j];
-                v[u] = va ? va[j] : (uint8_t)1;
-            }
-        }
-    }
-    // the slot is marked invalid: mask false, or a negative id in an int32 graph
-    __device__ __forceinline__ bool marked(int u) const {
-        if constexpr (I32) return y[u] < 0;
-        else return v[u] == 0;
-    }
-};
-
 template <typename T, int D, int U>
 __global__ void __launch_bounds__(WAVES * SSA_WAVE)
 apply_fwd_kernel(ApplyP p) {
@@ -289,65 +165,6 @@ apply_fwd_kernel(ApplyP p) {
     }
 }
 
-// ---------------------------------------------------------------- rows beyond LDS
-// Rows of more than APPLY_KLDS slots (whose scores do not fit a wave's share
-// of LDS): nothing is kept per slot.  The scores are computed again in each
-// pass over the row (same products, same order, so the same values): first
-// the softmax maximum and sum online (a slot raising the maximum rescales the
-// sum), then the weights, whose arithmetic is the kernels' above.
-constexpr int APPLY_KLDS = 4096;
-
-template <typename T, int VEC, int LPR>
-struct LongRow {
-    const ApplyP &p;
-    int64_t row;
-    const T *kb, *vb;
-    const int64_t *nb;
-    const uint8_t *va;
-    int lofs;
-    // key id of slot j, -1 when masked or out of range
-    __device__ int id(int j, bool *marked = nullptr) const {
-        const int64_t x = p.nb32 ? (int64_t)p.nb32[row * p.K + j] : nb[j];
-        const bool mk = p.nb32 ? x < 0 : (va ? va[j] == 0 : false);
-        if (marked) *marked = mk;
-        return (!mk && x >= 0 && x < p.M) ? (int)x : -1;
-    }
-    // score of slot j (key id x, -1: -inf), every lane of the slot's group
-    __device__ float score(const float (&qf)[VEC], int x) const {
-        float kf[VEC];
-        load_vec<T, VEC>(kb + (int64_t)(x < 0 ? 0 : x) * p.ksn + lofs, kf);
-        float part = 0.f;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) part = fmaf(qf[e], kf[e], part);
-#pragma unroll
-        for (int o = LPR / 2; o > 0; o >>= 1) part += __shfl_xor(part, o, SSA_WAVE);
-        return x >= 0 ? part * p.scale : -INFINITY;
-    }
-    // dout . v of key x (row 0 for -1), every lane of the slot's group
-    __device__ float dotv(const float (&dof)[VEC], int x) const {
-        float vf[VEC];
-        load_vec<T, VEC>(vb + (int64_t)(x < 0 ? 0 : x) * p.vsn + lofs, vf);
-        float part = 0.f;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) part = fmaf(dof[e], vf[e], part);
-#pragma unroll
-        for (int o = LPR / 2; o > 0; o >>= 1) part += __shfl_xor(part, o, SSA_WAVE);
-        return part;
-    }
-};
-
-// online softmax statistics of one lane group, then merged over the wave
-__device__ __forceinline__ void online_add(float s, float &m, float &l) {
-    if (s == -INFINITY) return;
-    if (s > m) { l = l * expf(m - s) + 1.f; m = s; }
-    else l += expf(s - m);
-}
-
-__device__ __forceinline__ void online_merge(bool lead, float m, float l, float &mm, float &ll) {
-    mm = wave_max(lead ? m : -INFINITY);
-    ll = wave_sum((lead && m != -INFINITY) ? l * expf(m - mm) : 0.f);
-}
-
 template <typename T, int D>
 __global__ void __launch_bounds__(WAVES * SSA_WAVE)
 apply_fwd_long_kernel(ApplyP p) {
@@ -432,96 +249,6 @@ apply_fwd_long_kernel(ApplyP p) {
 //    go through one v_dot2 per element: {p_j, p_j'} . {v_j[e], v_j'[e]},
 //    with the element pairs gathered by v_perm;
 //  * rows are addressed by 32-bit byte offsets from a wave-uniform base.
-template <typename T> struct Dot2;
-template <> struct Dot2<bf16_t> {
-    typedef __bf16 __attribute__((ext_vector_type(2))) v2;
-    static __device__ __forceinline__ float dot(uint32_t a, uint32_t b, float c) {
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2, a), __builtin_bit_cast(v2, b),
-                                               c, false);
-    }
-    // two bf16-exact fp32 values as a pair (a low, b high): their upper halves
-    static __device__ __forceinline__ uint32_t pack(float a, float b) {
-        return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
-    }
-    static __device__ __forceinline__ uint32_t bits(float v) { return f32_to_bf16_bits(v); }
-};
-template <> struct Dot2<f16_t> {
-    typedef _Float16 __attribute__((ext_vector_type(2))) v2;
-    static __device__ __forceinline__ float dot(uint32_t a, uint32_t b, float c) {
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(v2, a), __builtin_bit_cast(v2, b), c,
-                                      false);
-    }
-    static __device__ __forceinline__ uint32_t pack(float a, float b) {
-        const v2 h = {(_Float16)a, (_Float16)b};       // exact: both are fp16 values
-        return __builtin_bit_cast(uint32_t, h);
-    }
-    static __device__ __forceinline__ uint32_t bits(float v) {
-        const _Float16 h = (_Float16)v;
-        return (uint32_t)__builtin_bit_cast(uint16_t, h);
-    }
-};
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-    // every source lane of these patterns exists: old (0) is never used, and
-    // an identity old lets the move fold into the add as a DPP operand
-    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF,
-                                                          false));
-}
-
-// sum over the L lanes of each aligned group (L a power of two <= 32); every
-// lane of the group gets the sum
-template <int L>
-__device__ __forceinline__ float group_sum(float v) {
-    if constexpr (L >= 16) v = dpp_add<0x140>(v);   // row mirror
-    if constexpr (L >= 8) v = dpp_add<0x141>(v);    // row half mirror
-    if constexpr (L >= 2) v = dpp_add<0xB1>(v);     // quad perm [1,0,3,2]
-    if constexpr (L >= 4) v = dpp_add<0x4E>(v);     // quad perm [2,3,0,1]
-    if constexpr (L >= 32) v += __shfl_xor(v, 16, SSA_WAVE);
-    return v;
-}
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-
-// Reduce U per-lane partials (one per row) over the 2U lanes of a row group
-// by a butterfly: at each step a lane pair splits its rows, each lane sending
-// the half it drops and adding the half it keeps (row mirror, half mirror,
-// quad swaps as the pairings).  Afterwards lanes li and li ^ 1 both hold the
-// total of row r = 4 [li >= 8] + 2 [li & 4] + [li & 2] (U = 8), or
-// r = 2 [li & 4] + [li & 2] (U = 4).
-template <int U>
-__device__ __forceinline__ float butterfly_rows(float (&v)[U], int li) {
-    static_assert(U == 4 || U == 8, "butterfly over 8 or 16 lanes");
-    float w[4];
-    if constexpr (U == 8) {
-        const bool hi = li >= 8;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float send = hi ? v[k] : v[k + 4], keep = hi ? v[k + 4] : v[k];
-            w[k] = keep + dpp_move<0x140>(send);        // row mirror: li <-> 15 - li
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) w[k] = v[k];
-    }
-    float x[2];
-    {
-        const bool hi = (li & 4) != 0;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const float send = hi ? w[k] : w[k + 2], keep = hi ? w[k + 2] : w[k];
-            x[k] = keep + dpp_move<0x141>(send);        // half mirror: li <-> 7 - li (in 8)
-        }
-    }
-    const bool hi = (li & 2) != 0;
-    const float send = hi ? x[0] : x[1], keep = hi ? x[1] : x[0];
-    float y = keep + dpp_move<0x4E>(send);              // quad perm [2,3,0,1]: li ^ 2
-    return y + dpp_move<0xB1>(y);                       // quad perm [1,0,3,2]: li ^ 1
-}
-
 template <typename T, int D, int U>
 __global__ void __launch_bounds__(WAVES * SSA_WAVE)
 apply_fwd16_kernel(ApplyP p) {
@@ -711,11 +438,9 @@ apply_fwd16_kernel(ApplyP p) {
 
 // Backward: recompute p, then dp = dO.v, ds = p (dp - sum p dp), draw = ds*scale,
 // dq = sum draw k (direct store), dk += draw q, dv += p' dO (fp32 atomics).
-// DET (the deterministic backward's first pass): instead of the atomics, each
-// slot's draw and p' go to the workspace, and its key row's slot count and
-// largest |draw| and |p'| are raised (integer atomics, whose results do not
-// depend on their order), as are the largest |q| and |dout|.
-template <typename T, int D, bool DET>
+// The form without a workspace (ssa_sparse_gather_attention_bwd); ssa_grad.hip
+// sums the key rows without atomics and is many times faster.
+template <typename T, int D>
 __global__ void __launch_bounds__(WAVES * SSA_WAVE)
 apply_bwd_kernel(ApplyP p) {
     using G = Geo<T, D>;
@@ -799,21 +524,6 @@ apply_bwd_kernel(ApplyP p) {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
-    if (DET) {
-        // the largest |q| and |dout| bound every slot's contributions
-        float qm = 0.f, dm = 0.f;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) {
-            qm = fmaxf(qm, fabsf(qf[e]));
-            dm = fmaxf(dm, fabsf(dof[e]));
-        }
-        qm = wave_max(qm);
-        dm = wave_max(dm);
-        if (lane == 0) {
-            atomicMax(&p.gmax[0], __float_as_uint(qm));
-            atomicMax(&p.gmax[1], __float_as_uint(dm));
-        }
-    }
     float dqa[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) dqa[e] = 0.f;
@@ -821,10 +531,7 @@ apply_bwd_kernel(ApplyP p) {
         const int j = j0 + sub;
         if (j >= p.K) continue;
         int64_t x = nb[j];
-        if (x < 0 || x >= p.M) {
-            if (DET && li == 0) { p.wdraw[row * p.K + j] = 0.f; p.wpw[row * p.K + j] = 0.f; }
-            continue;
-        }
+        if (x < 0 || x >= p.M) continue;
         const float pj = sc[j];
         const float draw = pj * (dpv[j] - pdp) * p.scale;
         float mask = 1.f;
@@ -833,25 +540,13 @@ apply_bwd_kernel(ApplyP p) {
         float kf[VEC];
         load_vec<T, VEC>(kb + x * p.ksn + lofs, kf);
         const int64_t kr = ((int64_t)b * p.Hkv + g) * p.M + x;
-        if (DET) {
-            if (li == 0) {
-                p.wdraw[row * p.K + j] = draw;
-                p.wpw[row * p.K + j] = pw;
-                atomicAdd(&p.kcnt[kr], 1u);
-                atomicMax(&p.kmaxd[kr], __float_as_uint(fabsf(draw)));
-                atomicMax(&p.kmaxp[kr], __float_as_uint(fabsf(pw)));
-            }
+        float *dkr = p.dk + kr * p.d + lofs;
+        float *dvr = p.dv + kr * p.d + lofs;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) dqa[e] = fmaf(draw, kf[e], dqa[e]);
-        } else {
-            float *dkr = p.dk + kr * p.d + lofs;
-            float *dvr = p.dv + kr * p.d + lofs;
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) {
-                dqa[e] = fmaf(draw, kf[e], dqa[e]);
-                if (live && draw != 0.f) unsafeAtomicAdd(dkr + e, draw * qf[e]);
-                if (live && pw != 0.f) unsafeAtomicAdd(dvr + e, pw * dof[e]);
-            }
+        for (int e = 0; e < VEC; ++e) {
+            dqa[e] = fmaf(draw, kf[e], dqa[e]);
+            if (live && draw != 0.f) unsafeAtomicAdd(dkr + e, draw * qf[e]);
+            if (live && pw != 0.f) unsafeAtomicAdd(dvr + e, pw * dof[e]);
         }
     }
 #pragma unroll
@@ -868,7 +563,7 @@ apply_bwd_kernel(ApplyP p) {
 // Backward of rows beyond LDS: the softmax statistics online, then
 // sum p dp, then each slot's draw and p' (the arithmetic of apply_bwd_kernel,
 // with the scores and dout . v computed again in each pass).
-template <typename T, int D, bool DET>
+template <typename T, int D>
 __global__ void __launch_bounds__(WAVES * SSA_WAVE)
 apply_bwd_long_kernel(ApplyP p) {
     using G = Geo<T, D>;
@@ -897,20 +592,6 @@ apply_bwd_long_kernel(ApplyP p) {
     for (int e = 0; e < VEC; ++e) {
         dof[e] = live ? dorow[e] : 0.f;
         qf[e] = live ? qf[e] : 0.f;
-    }
-    if (DET) {
-        float qm = 0.f, dm = 0.f;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) {
-            qm = fmaxf(qm, fabsf(qf[e]));
-            dm = fmaxf(dm, fabsf(dof[e]));
-        }
-        qm = wave_max(qm);
-        dm = wave_max(dm);
-        if (lane == 0) {
-            atomicMax(&p.gmax[0], __float_as_uint(qm));
-            atomicMax(&p.gmax[1], __float_as_uint(dm));
-        }
     }
     // the ids are read from the graph in each pass (the graph's validity and
     // range rules of the forward; the backward takes int64 ids only)
@@ -942,10 +623,7 @@ apply_bwd_long_kernel(ApplyP p) {
         const int j = j0 + sub;
         if (j >= p.K) continue;
         const int64_t xr = R.nb[j];
-        if (xr < 0 || xr >= p.M) {
-            if (DET && li == 0) { p.wdraw[row * p.K + j] = 0.f; p.wpw[row * p.K + j] = 0.f; }
-            continue;
-        }
+        if (xr < 0 || xr >= p.M) continue;
         const int x = R.id(j);
         const float pj = expf(R.score(qf, x) - mm) / ll;
         const float mask = mask_of(j);
@@ -954,25 +632,13 @@ apply_bwd_long_kernel(ApplyP p) {
         float kf[VEC];
         load_vec<T, VEC>(R.kb + xr * p.ksn + R.lofs, kf);
         const int64_t kr = ((int64_t)b * p.Hkv + g) * p.M + xr;
-        if (DET) {
-            if (li == 0) {
-                p.wdraw[row * p.K + j] = draw;
-                p.wpw[row * p.K + j] = pw;
-                atomicAdd(&p.kcnt[kr], 1u);
-                atomicMax(&p.kmaxd[kr], __float_as_uint(fabsf(draw)));
-                atomicMax(&p.kmaxp[kr], __float_as_uint(fabsf(pw)));
-            }
+        float *dkr = p.dk + kr * p.d + R.lofs;
+        float *dvr = p.dv + kr * p.d + R.lofs;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) dqa[e] = fmaf(draw, kf[e], dqa[e]);
-        } else {
-            float *dkr = p.dk + kr * p.d + R.lofs;
-            float *dvr = p.dv + kr * p.d + R.lofs;
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) {
-                dqa[e] = fmaf(draw, kf[e], dqa[e]);
-                if (live && draw != 0.f) unsafeAtomicAdd(dkr + e, draw * qf[e]);
-                if (live && pw != 0.f) unsafeAtomicAdd(dvr + e, pw * dof[e]);
-            }
+        for (int e = 0; e < VEC; ++e) {
+            dqa[e] = fmaf(draw, kf[e], dqa[e]);
+            if (live && draw != 0.f) unsafeAtomicAdd(dkr + e, draw * qf[e]);
+            if (live && pw != 0.f) unsafeAtomicAdd(dvr + e, pw * dof[e]);
         }
     }
 #pragma unroll
@@ -984,98 +650,6 @@ apply_bwd_long_kernel(ApplyP p) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) dqr[e] = dqa[e];
     }
-}
-
-// ---- deterministic backward: fixed-point sums
-// A key row's gradient is a sum over the (query row, slot) pairs that hold it.
-// Its terms are rounded to a fixed-point grid of that key row and summed as
-// 64-bit integers, whose sum does not depend on the order the atomics land
-// in; the grid 2^-s is the finest for which the sum cannot overflow: count x
-// largest weight x largest |q| (or |dout|) below 2^(61 - s).  Returns -1
-// when the key row has no term, -2 when a bound is not finite.
-__device__ __forceinline__ int fx_shift(uint32_t cnt, uint32_t wbits, uint32_t xbits) {
-    const double bound = (double)cnt * (double)__uint_as_float(wbits) * (double)__uint_as_float(xbits);
-    if (!(bound == bound) || bound > 1e300) return -2;
-    if (!(bound > 0.0)) return -1;
-    int e = 0;
-    (void)frexp(bound, &e);                 // bound < 2^e
-    return 61 - e;
-}
-
-__device__ __forceinline__ unsigned long long fx_of(float c, int s) {
-    return (unsigned long long)(long long)rint(ldexp((double)c, s));
-}
-
-// second pass: per query row, each slot's terms draw * q and p' * dout added
-// to its key row's fixed-point sums
-template <typename T, int D>
-__global__ void __launch_bounds__(WAVES * SSA_WAVE)
-apply_bwd_fx_kernel(ApplyP p) {
-    using G = Geo<T, D>;
-    constexpr int VEC = G::VEC, LPR = G::LPR, RPI = G::RPI;
-    const int64_t blk = xcd_logical_block(blockIdx.x, p.nblocks);
-    if (blk >= p.nblocks) return;
-    const int wid = threadIdx.x / SSA_WAVE;
-    const int64_t row = blk * WAVES + wid;
-    if (row >= p.rows) return;
-    const int lane = lane_id();
-    const int sub = lane / LPR, li = lane % LPR;
-    const int n = (int)(row % p.N);
-    const int64_t bh = row / p.N;
-    const int h = (int)(bh % p.Hq);
-    const int b = (int)(bh / p.Hq);
-    const int g = h / p.rep;
-    const T *qrow = (const T *)p.q + b * p.qsb + h * p.qsh + (int64_t)n * p.qsn;
-    const int64_t *nb = p.nb + row * p.K;
-    const bool live = li * VEC < p.d;
-    const int lofs = live ? li * VEC : 0;
-    const float *dorow = p.dout + row * p.d + lofs;
-    float qf[VEC], dof[VEC];
-    load_vec<T, VEC>(qrow + lofs, qf);
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-        dof[e] = live ? dorow[e] : 0.f;
-        qf[e] = live ? qf[e] : 0.f;
-    }
-    const uint32_t qmax = p.gmax[0], dmax = p.gmax[1];
-    for (int j0 = 0; j0 < p.K; j0 += RPI) {
-        const int j = j0 + sub;
-        if (j >= p.K) continue;
-        const int64_t x = nb[j];
-        if (x < 0 || x >= p.M) continue;
-        const float draw = p.wdraw[row * p.K + j], pw = p.wpw[row * p.K + j];
-        const int64_t kr = ((int64_t)b * p.Hkv + g) * p.M + x;
-        const uint32_t cnt = p.kcnt[kr];
-        const int sk = fx_shift(cnt, p.kmaxd[kr], qmax);
-        const int sv = fx_shift(cnt, p.kmaxp[kr], dmax);
-        unsigned long long *ak = p.acck + kr * p.d + lofs;
-        unsigned long long *av = p.accv + kr * p.d + lofs;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) {
-            if (live && draw != 0.f && sk >= 0) atomicAdd(ak + e, fx_of(draw * qf[e], sk));
-            if (live && pw != 0.f && sv >= 0) atomicAdd(av + e, fx_of(pw * dof[e], sv));
-        }
-    }
-}
-
-// last pass: dk += sum * 2^-s, dv likewise, per element (NaN where a bound
-// was not finite)
-__global__ void __launch_bounds__(256) apply_bwd_finish_kernel(ApplyP p, int64_t total) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= total) return;
-    const int64_t kr = i / p.d;
-    const uint32_t cnt = p.kcnt[kr];
-    const int sk = fx_shift(cnt, p.kmaxd[kr], p.gmax[0]);
-    const int sv = fx_shift(cnt, p.kmaxp[kr], p.gmax[1]);
-    if (sk >= 0) p.dk[i] += (float)ldexp((double)(long long)p.acck[i], -sk);
-    else if (sk == -2) p.dk[i] = __builtin_nanf("");
-    if (sv >= 0) p.dv[i] += (float)ldexp((double)(long long)p.accv[i], -sv);
-    else if (sv == -2) p.dv[i] = __builtin_nanf("");
-}
-
-__global__ void __launch_bounds__(256) apply_zero_kernel(uint32_t *w, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
-        w[i] = 0u;
 }
 
 // The 16-bit path needs weights in the value dtype, 16-byte aligned rows,
@@ -1105,41 +679,18 @@ int launch_apply(const ApplyP &p, hipStream_t st, bool bwd) {
         SSA_CHECK_LAUNCH();
         return SSA_OK;
     }
-    if (lng && !p.wdraw) {
-        hipLaunchKernelGGL((apply_bwd_long_kernel<T, D, false>), dim3((unsigned)grid),
+    if (lng) {
+        hipLaunchKernelGGL((apply_bwd_long_kernel<T, D>), dim3((unsigned)grid),
                            dim3(WAVES * SSA_WAVE), 0, st, p);
         SSA_CHECK_LAUNCH();
         return SSA_OK;
     }
-    if (bwd && p.wdraw) {
-        // deterministic: rows (dq, weights, bounds), fixed-point sums, finish
-        if (lng) {
-            hipLaunchKernelGGL((apply_bwd_long_kernel<T, D, true>), dim3((unsigned)grid),
-                               dim3(WAVES * SSA_WAVE), 0, st, p);
-        } else {
-            const size_t lds = (size_t)WAVES * 2 * p.K * sizeof(float);
-            if (lds > 65536)
-                SSA_CHECK_HIP(hipFuncSetAttribute((const void *)apply_bwd_kernel<T, D, true>,
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                  (int)lds));
-            hipLaunchKernelGGL((apply_bwd_kernel<T, D, true>), dim3((unsigned)grid),
-                               dim3(WAVES * SSA_WAVE), lds, st, p);
-        }
-        SSA_CHECK_LAUNCH();
-        hipLaunchKernelGGL((apply_bwd_fx_kernel<T, D>), dim3((unsigned)grid),
-                           dim3(WAVES * SSA_WAVE), 0, st, p);
-        SSA_CHECK_LAUNCH();
-        const int64_t total = (int64_t)p.B * p.Hkv * p.M * p.d;
-        if (total > 0) {
-            hipLaunchKernelGGL(apply_bwd_finish_kernel, dim3((unsigned)ceil_div(total, 256)),
-                               dim3(256), 0, st, p, total);
-        }
-    } else if (bwd) {
+    if (bwd) {
         const size_t lds = (size_t)WAVES * 2 * p.K * sizeof(float);
         if (lds > 65536)
-            SSA_CHECK_HIP(hipFuncSetAttribute((const void *)apply_bwd_kernel<T, D, false>,
+            SSA_CHECK_HIP(hipFuncSetAttribute((const void *)apply_bwd_kernel<T, D>,
                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((apply_bwd_kernel<T, D, false>), dim3((unsigned)grid),
+        hipLaunchKernelGGL((apply_bwd_kernel<T, D>), dim3((unsigned)grid),
                            dim3(WAVES * SSA_WAVE), lds, st, p);
     } else {
         const size_t lds = (size_t)WAVES * 2 * p.K * sizeof(float);
@@ -1193,50 +744,6 @@ int dispatch_d(const ApplyP &p, int d, hipStream_t st, bool bwd) {
     }
 }
 
-int check_view(const ssa_tensor4 &t, int dtype, const char *name) {
-    if (!t.ptr) { ssa_set_error("%s: null pointer", name); return SSA_E_ARG; }
-    if (t.dtype != dtype) { ssa_set_error("%s: dtype mismatch", name); return SSA_E_ARG; }
-    return SSA_OK;
-}
-
-int apply_common(const ssa_apply_args *a, ApplyP &p) {
-    SSA_CHECK_ARG(a != nullptr, "sparse_gather_attention: null args");
-    SSA_CHECK_ARG(a->B >= 0 && a->Hq > 0 && a->Hkv > 0 && a->N >= 0 && a->M > 0 && a->K >= 0,
-                  "sparse_gather_attention: bad sizes B=%d Hq=%d Hkv=%d N=%d M=%d K=%d", a->B,
-                  a->Hq, a->Hkv, a->N, a->M, a->K);
-    SSA_CHECK_ARG(a->Hq % a->Hkv == 0, "sparse_gather_attention: Hq %% Hkv != 0");
-    SSA_CHECK_ARG((int64_t)a->B * a->Hq * a->N * a->K < ((int64_t)1 << 62),
-                  "sparse_gather_attention: too many slots");
-    SSA_CHECK_ARG(a->q.dtype >= 0 && a->q.dtype <= 2, "sparse_gather_attention: bad dtype");
-    int rc;
-    if ((rc = check_view(a->q, a->q.dtype, "q"))) return rc;
-    if ((rc = check_view(a->k, a->q.dtype, "k"))) return rc;
-    if ((rc = check_view(a->v, a->q.dtype, "v"))) return rc;
-    SSA_CHECK_ARG((a->neighbors != nullptr || a->neighbors32 != nullptr) && a->out != nullptr,
-                  "sparse_gather_attention: null");
-    SSA_CHECK_ARG(a->dropout_p >= 0.f && a->dropout_p < 1.f, "dropout p must be in [0, 1)");
-    p = ApplyP{};
-    p.B = a->B; p.Hq = a->Hq; p.Hkv = a->Hkv; p.N = a->N; p.M = a->M; p.K = a->K;
-    p.rep = a->Hq / a->Hkv;
-    p.d = a->d;
-    p.q = a->q.ptr; p.k = a->k.ptr; p.v = a->v.ptr;
-    p.qsb = a->q.sb; p.qsh = a->q.sh; p.qsn = a->q.sn;
-    p.ksb = a->k.sb; p.ksh = a->k.sh; p.ksn = a->k.sn;
-    p.vsb = a->v.sb; p.vsh = a->v.sh; p.vsn = a->v.sn;
-    p.nb = a->neighbors; p.valid = a->valid; p.nb32 = a->neighbors32;
-    p.row_inv = a->row_invalid;
-    p.scale = a->scale; p.fp32w = a->fp32_weights;
-    p.drop_p = a->dropout_p;
-    // inverted dropout scales kept weights by 1 / (1 - p), the keep rate taken
-    // in double and rounded to fp32 as torch's dropout divides its noise
-    p.drop_scale = a->dropout_p > 0.f ? 1.f / (float)(1.0 - (double)a->dropout_p) : 1.f;
-    p.seed = a->seed;
-    p.out = a->out; p.osb = a->out_sb; p.osh = a->out_sh; p.osn = a->out_sn;
-    p.rows = (int64_t)a->B * a->Hq * a->N;
-    p.nblocks = ceil_div(p.rows, WAVES);
-    return SSA_OK;
-}
-
 int run_apply(const ApplyP &p, int dtype, int d, hipStream_t st, bool bwd) {
     if (p.rows == 0) return SSA_OK;
     switch (dtype) {
@@ -1271,32 +778,6 @@ int bwd_common(const ssa_apply_bwd_args *a, ApplyP &p) {
     return SSA_OK;
 }
 
-int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
-
-// workspace of the deterministic backward: the per-slot weights, then (zeroed
-// together) the key rows' counts and bounds, the two maxima and the sums
-struct DetLayout {
-    int64_t wdraw, wpw, zero_at, kcnt, kmaxd, kmaxp, gmax, acck, accv, total;
-};
-
-DetLayout det_layout(const ApplyP &p) {
-    DetLayout L{};
-    const int64_t slots = p.rows * p.K, keys = (int64_t)p.B * p.Hkv * p.M;
-    int64_t o = 0;
-    auto take = [&](int64_t bytes) { const int64_t at = o; o += align256(bytes); return at; };
-    L.wdraw = take(slots * 4);
-    L.wpw = take(slots * 4);
-    L.zero_at = o;
-    L.kcnt = take(keys * 4);
-    L.kmaxd = take(keys * 4);
-    L.kmaxp = take(keys * 4);
-    L.gmax = take(8);
-    L.acck = take(keys * p.d * 8);
-    L.accv = take(keys * p.d * 8);
-    L.total = o;
-    return L;
-}
-
 }  // namespace
 
 extern "C" int ssa_sparse_gather_attention_bwd(const ssa_apply_bwd_args *a, void *stream) {
@@ -1304,40 +785,4 @@ extern "C" int ssa_sparse_gather_attention_bwd(const ssa_apply_bwd_args *a, void
     const int rc = bwd_common(a, p);
     if (rc) return rc;
     return run_apply(p, a->fwd.q.dtype, a->fwd.d, (hipStream_t)stream, true);
-}
-
-extern "C" int64_t ssa_sparse_gather_attention_bwd_det_workspace_bytes(const ssa_apply_bwd_args *a) {
-    ApplyP p;
-    const int rc = bwd_common(a, p);
-    if (rc) return rc;
-    return det_layout(p).total;
-}
-
-extern "C" int ssa_sparse_gather_attention_bwd_det(const ssa_apply_bwd_args *a, void *workspace,
-                                                   int64_t workspace_bytes, void *stream) {
-    ApplyP p;
-    const int rc = bwd_common(a, p);
-    if (rc) return rc;
-    const DetLayout L = det_layout(p);
-    SSA_CHECK_ARG(workspace != nullptr && workspace_bytes >= L.total,
-                  "sparse_gather_attention_bwd_det: workspace of %lld bytes, %lld needed",
-                  (long long)workspace_bytes, (long long)L.total);
-    SSA_CHECK_ARG((uintptr_t)workspace % 256 == 0,
-                  "sparse_gather_attention_bwd_det: workspace must be 256-byte aligned");
-    if (p.rows == 0) return SSA_OK;
-    char *ws = (char *)workspace;
-    p.wdraw = (float *)(ws + L.wdraw);
-    p.wpw = (float *)(ws + L.wpw);
-    p.kcnt = (uint32_t *)(ws + L.kcnt);
-    p.kmaxd = (uint32_t *)(ws + L.kmaxd);
-    p.kmaxp = (uint32_t *)(ws + L.kmaxp);
-    p.gmax = (uint32_t *)(ws + L.gmax);
-    p.acck = (unsigned long long *)(ws + L.acck);
-    p.accv = (unsigned long long *)(ws + L.accv);
-    const hipStream_t st = (hipStream_t)stream;
-    const int64_t nz = (L.total - L.zero_at) / 4;
-    hipLaunchKernelGGL(apply_zero_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(nz, 256), 4096)),
-                       dim3(256), 0, st, (uint32_t *)(ws + L.zero_at), nz);
-    SSA_CHECK_LAUNCH();
-    return run_apply(p, a->fwd.q.dtype, a->fwd.d, st, true);
 }

@@ -230,16 +230,14 @@ class _GatherAttention(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
-        # under torch.use_deterministic_algorithms(True) the backward whose
-        # dK / dV sums are fixed-point (the same bits on every run); else the
-        # faster one that adds them with fp32 atomics
+        # under torch.use_deterministic_algorithms(True) the key rows' sums do
+        # not depend on the order of their terms: the same bits on every run
         q, k, v, neighbors, valid = ctx.saved_tensors
         scale, fp32w, dropout_p, seed = ctx.cfg
-        dq, dk, dv = _lib.gather_attention_bwd(q, k, v, neighbors, valid, scale, fp32w,
-                                               dropout_p, seed, dout,
-                                               deterministic=torch.are_deterministic_algorithms_enabled())
-        return (dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), None, None, None, None, None,
-                None, None)
+        dq, dk, dv = _lib.gather_attention_grad(
+            q, k, v, neighbors, valid, scale, fp32w, dropout_p, seed, dout,
+            deterministic=torch.are_deterministic_algorithms_enabled())
+        return dq, dk, dv, None, None, None, None, None, None, None
 
 
 def sparse_gather_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
