@@ -97,6 +97,8 @@ struct Dims {
                        // hash or aux pass, aux rows for every head, split hyperplanes
     int cbits;         // width of the cut entries' size and cutoff fields
     int swaves;        // rows (waves) per select workgroup, as many as its LDS allows
+    int dense;         // every key scored once, candidates as bitmaps (ssa_graph_dense.h)
+    int Ms, nw;        // dense: codes per score row, 64-key words per bitmap
 };
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -1550,6 +1552,13 @@ struct SelP {
     int NA;
     int perm_bytes;        // size of the permutation array (B*Hkv*R*M*4 < 2^31)
     int64_t nblocks;
+    // dense form
+    const uint32_t *S32;   // score rows as 32-bit pairs
+    const uint64_t *lbits; // bucket bitmaps
+    const int32_t *lmax;   // largest member of each bucket's list
+    const uint32_t *knorm; // max |k|^2 per (batch, kv head), float bits
+    int Ms, nw;
+    uint32_t magN, magHq, magRep, magNS;   // ceil(2^32 / N) and so on
 };
 
 __device__ __forceinline__ void bm_set(uint32_t *bm, int v) { atomicOr(&bm[v >> 5], 1u << (v & 31)); }
@@ -2534,6 +2543,9 @@ select_kernel(SelP p) {
 
     full_merge_emit(bm, p, n, row, f, (int32_t *)ckey, sel_buf_words(p.words, CAP));
 }
+
+// ------------------------------------------------------------------ dense form
+#include "ssa_graph_dense.h"
 
 // ------------------------------------------------------------------ exact top-k replay
 // A row whose kk-th kept score is tied, or (LSH mode) whose selected scores are
@@ -3522,7 +3534,7 @@ struct Layout {
     int64_t kid, qid, perm, bstart, bsize, sorttmp, sid, rnk, smin, inv, cut, srix, cnt, off,
         cur,
         qlist, tiles, ntiles, tcnt, kbase, S,
-        tie_list, tie_count, aux, psplit, knorm, kpart, rpscr, rpw, ctab, total;
+        tie_list, tie_count, aux, psplit, knorm, kpart, rpscr, rpw, ctab, lbits, lmax, total;
 };
 
 int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
@@ -3539,22 +3551,28 @@ Layout plan(const Dims &D) {
     L.bstart = take(D.BK * D.R * D.NB * 4);
     L.bsize = take(D.BK * D.R * D.NB * 4);
     L.sorttmp = take(ssa_sort_tmp_bytes((int)(D.BK * D.R), D.M));
-    L.sid = take(D.BK * D.R * D.M * 4);
-    L.rnk = take(D.BK * D.R * D.M * 4);
-    L.smin = take(D.BK * D.R * D.M * 4);
-    L.inv = take(D.BK * D.R * D.M * 4);
-    L.cut = take(nbh * D.N * D.nlists * 16);
-    L.srix = take(nbh * D.N * D.nlists * 4);
-    L.cnt = take(ninst * D.NB * 4);
-    L.off = take(ninst * D.NB * 4);
-    L.cur = take(ninst * ceil_div(D.N, 256) * D.NB * 4);   // per-block counts / bases
-    L.qlist = take(ninst * D.N * 4);
-    // one 16-byte slot per block of the rescore grid (a multiple of 8)
-    L.tiles = take(8 * ceil_div(ninst * (ceil_div(D.N, TQ) + D.NB), 8) * 16);
-    L.ntiles = take(4);
-    L.tcnt = take(ninst * 4);
-    L.kbase = take((nbh / D.rep + 2) * D.R * D.NS * D.rep * 4);
-    L.S = take(nbh * D.N * D.nlists * D.Cs * 2);
+    if (D.dense) {
+        L.S = take(nbh * D.N * D.Ms * 2);
+        L.lbits = take(D.BK * D.R * D.NB * (int64_t)D.nw * 8);
+        L.lmax = take(D.BK * D.R * D.NB * 4);
+    } else {
+        L.sid = take(D.BK * D.R * D.M * 4);
+        L.rnk = take(D.BK * D.R * D.M * 4);
+        L.smin = take(D.BK * D.R * D.M * 4);
+        L.inv = take(D.BK * D.R * D.M * 4);
+        L.cut = take(nbh * D.N * D.nlists * 16);
+        L.srix = take(nbh * D.N * D.nlists * 4);
+        L.cnt = take(ninst * D.NB * 4);
+        L.off = take(ninst * D.NB * 4);
+        L.cur = take(ninst * ceil_div(D.N, 256) * D.NB * 4);   // per-block counts / bases
+        L.qlist = take(ninst * D.N * 4);
+        // one 16-byte slot per block of the rescore grid (a multiple of 8)
+        L.tiles = take(8 * ceil_div(ninst * (ceil_div(D.N, TQ) + D.NB), 8) * 16);
+        L.ntiles = take(4);
+        L.tcnt = take(ninst * 4);
+        L.kbase = take((nbh / D.rep + 2) * D.R * D.NS * D.rep * 4);
+        L.S = take(nbh * D.N * D.nlists * D.Cs * 2);
+    }
     L.tie_list = take(D.BH * D.N * 4);
     L.tie_count = take(4);
     L.aux = take((D.fused ? D.BH : nbh) * D.N * (D.G + 3) * 4);
@@ -3574,6 +3592,17 @@ Layout plan(const Dims &D) {
     }
     L.total = o;
     return L;
+}
+
+// Whether the build takes the dense form (ssa_graph_dense.h): a graph, keys
+// within a select row's registers, lists within a wave's lanes, a round's
+// bitmaps within LDS, and lists that hold in all at least as many members as
+// there are keys (below that the list form reads fewer scores).
+bool dense_form(const Dims &D, const ssa_graph_args *a) {
+    const int64_t nw = ceil_div(D.M, 64);
+    const int64_t members = (int64_t)D.nlists * std::min<int64_t>(D.C, ceil_div(D.M, D.NB));
+    return a->mode == SSA_GRAPH_FULL && D.M <= DN_MAX_KEYS && D.nlists <= DN_MAX_LISTS &&
+           D.NB * (nw * 8 + 4) <= DN_BITS_LDS && members * DN_NUM >= D.M * (int64_t)DN_DEN;
 }
 
 Layout plan(const Dims &D);
@@ -3717,10 +3746,24 @@ int make_dims(const ssa_graph_args *a, Dims &D, bool need_q = true, int64_t ws_c
         const int64_t tb = D.BK * D.R * D.NB * (int64_t)((D.M + 31) / 32) * 8;
         D.ctab = a->causal && tb <= (ws_cap > 0 ? ws_cap / 16 : ((int64_t)256 << 20)) ? 1 : 0;
     }
-    int64_t nbh = ((int64_t)8 << 30) / per_bh;
-    if (nbh < 1) nbh = 1;
-    if (nbh > D.BH) nbh = D.BH;
-    D.nbh_chunk = (int)nbh;
+    D.Ms = (int)ceil_div(D.M, DN_BLK) * DN_BLK;
+    if (D.Ms % 1024 == 0) D.Ms += DN_BLK;
+    D.nw = (int)ceil_div(D.M, 64);
+    auto chunk_heads = [&]() {
+        const int64_t per = D.dense ? (int64_t)D.N * D.Ms * 2 : per_bh;
+        D.nbh_chunk = (int)std::max<int64_t>(1, std::min(((int64_t)8 << 30) / per, D.BH));
+    };
+    D.dense = dense_form(D, a) ? 1 : 0;
+    chunk_heads();
+    if (ws_cap > 0 && D.dense) {
+        // the list form where the dense one does not fit with one head per chunk
+        Dims one = D;
+        one.nbh_chunk = 1;
+        if (plan(one).total > ws_cap) {
+            D.dense = 0;
+            chunk_heads();
+        }
+    }
     if (ws_cap > 0 && plan(D).total > ws_cap) {
         // the workspace grows with the chunk's head count: the largest count
         // in [1, nbh) that fits, by bisection
@@ -4181,11 +4224,12 @@ int launch_sort_aux(const Dims &D, const ssa_graph_args *a, const Layout &L, cha
     const QbP qp = qb_params(D, a, L, ws, 0, nbh);
     const int nseg = ssa_sort_seg_blocks(sa.rows, sa.n);
     const int nqb = (int)ceil_div(D.N, 256);
+    const int64_t nhist = D.dense ? 0 : (int64_t)qp.ninst * nqb;
     const size_t hl = std::max<size_t>((size_t)SEG_WAVES * seg_lds_words<uint16_t>() * 4,
                                        (size_t)D.NB * 4);
     SSA_CHECK_HIP(hipFuncSetAttribute((const void *)sort_seg_hist_kernel,
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)hl));
-    hipLaunchKernelGGL(sort_seg_hist_kernel, dim3((unsigned)(nseg + (int64_t)qp.ninst * nqb)),
+    hipLaunchKernelGGL(sort_seg_hist_kernel, dim3((unsigned)(nseg + nhist)),
                        dim3(256), hl, st, sa, qp, nseg, nqb);
     SSA_CHECK_LAUNCH();
     return SSA_OK;
@@ -4242,7 +4286,23 @@ int keys_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws
                                     false);
     }
     if (rc) return rc;
-    {
+    if (D.dense) {
+        LbP bp{};
+        bp.perm = (const int32_t *)(ws + L.perm);
+        bp.bstart = (const int32_t *)(ws + L.bstart);
+        bp.kid = (const uint16_t *)(ws + L.kid);
+        bp.bits = (uint64_t *)(ws + L.lbits);
+        bp.lmax = (int32_t *)(ws + L.lmax);
+        bp.M = D.M; bp.NB = D.NB; bp.C = D.C; bp.R = D.R; bp.nw = D.nw;
+        if (key_norm_in_hash(D, a)) {
+            bp.kpart = (const uint32_t *)(ws + L.kpart);
+            bp.knorm = (uint32_t *)(ws + L.knorm);
+            bp.kp_n = D.M / 16;
+        }
+        const size_t lds = (size_t)D.NB * (D.nw * 8 + 4);
+        hipLaunchKernelGGL(list_bits_kernel, dim3((unsigned)(D.BK * D.R)), dim3(1024), lds, st, bp);
+        SSA_CHECK_LAUNCH();
+    } else {
         LsP lp{};
         lp.perm = (const int32_t *)(ws + L.perm);
         lp.bstart = (const int32_t *)(ws + L.bstart);
@@ -4293,6 +4353,99 @@ int keys_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws
     return SSA_OK;
 }
 
+// The select's parameters that both forms share, for the head chunk
+// [bh0, bh0 + nbh)
+template <typename T>
+SelP select_common(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws, int64_t bh0,
+                   int nbh, bool mfma) {
+    SelP sp{};
+    sp.qid = (const uint16_t *)(ws + L.qid);
+    sp.perm = (const int32_t *)(ws + L.perm);
+    sp.bstart = (const int32_t *)(ws + L.bstart);
+    sp.bsize = (const int32_t *)(ws + L.bsize);
+    sp.mfma = mfma ? 1 : 0;
+    sp.nl_magic = (uint32_t)((((uint64_t)1 << 32) + D.nlists - 1) / D.nlists);
+    sp.q = a->q.ptr; sp.k = a->k.ptr;
+    sp.qsb = a->q.sb; sp.qsh = a->q.sh; sp.qsn = a->q.sn;
+    sp.ksb = a->k.sb; sp.ksh = a->k.sh; sp.ksn = a->k.sn;
+    sp.glob = a->glob;
+    sp.N = D.N; sp.M = D.M; sp.d = D.d; sp.R = D.R; sp.NS = D.NS; sp.NB = D.NB; sp.C = D.C;
+    sp.Cs = D.Cs;
+    sp.CPL = D.CPL; sp.nlists = D.nlists; sp.Hq = D.Hq; sp.Hkv = D.Hkv; sp.rep = D.rep;
+    sp.G = D.G; sp.kk = D.kk; sp.window = a->window; sp.causal = a->causal;
+    sp.cross = a->is_cross; sp.mode = a->mode; sp.total_k = a->total_k; sp.Kw = D.Kw;
+    sp.Kout = D.Kout; sp.bh0 = (int)bh0; sp.words = sel_bitmap_words(D.M);
+    sp.Call = D.Call; sp.rows = (int64_t)nbh * D.N; sp.rows_all = D.BH * D.N;
+    sp.out_idx = a->out_idx; sp.out_valid = a->out_valid; sp.ties = a->out_ties;
+    sp.out_idx32 = a->mode == SSA_GRAPH_FULL ? a->out_idx32 : nullptr;
+    sp.tie_list = (int32_t *)(ws + L.tie_list);
+    sp.tie_count = (int32_t *)(ws + L.tie_count);
+    sp.perm_bytes = (int)(D.BK * D.R * D.M * 4);
+    sp.cbits = D.cbits;
+    return sp;
+}
+
+// dense form: the codes of every (query, key) score of a head chunk
+template <typename T>
+int dense_scores(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws, SelP &sp,
+                 hipStream_t st) {
+    sp.S32 = (const uint32_t *)(ws + L.S);
+    sp.lbits = (const uint64_t *)(ws + L.lbits);
+    sp.lmax = (const int32_t *)(ws + L.lmax);
+    sp.knorm = (const uint32_t *)(ws + L.knorm);
+    sp.Ms = D.Ms; sp.nw = D.nw;
+    auto magic = [](int d) { return (uint32_t)((((uint64_t)1 << 32) + d - 1) / d); };
+    sp.magN = magic(D.N); sp.magHq = magic(D.Hq); sp.magRep = magic(D.rep); sp.magNS = magic(D.NS);
+    DnP dp{};
+    dp.q = a->q.ptr; dp.k = a->k.ptr;
+    dp.qsb = a->q.sb; dp.qsh = a->q.sh; dp.qsn = a->q.sn;
+    dp.ksb = a->k.sb; dp.ksh = a->k.sh; dp.ksn = a->k.sn;
+    dp.S = (uint32_t *)(ws + L.S);
+    dp.aux = sp.aux; dp.knorm = sp.knorm; dp.NA = sp.NA;
+    dp.N = D.N; dp.M = D.M; dp.Ms = D.Ms; dp.Hq = D.Hq; dp.Hkv = D.Hkv; dp.rep = D.rep;
+    dp.bh0 = sp.bh0; dp.nbh = (int)(sp.rows / D.N); dp.causal = a->causal ? 1 : 0; dp.d = D.d;
+    const bool mfma = sp.mfma != 0;
+    dp.qtiles = (int)ceil_div(D.N, mfma ? DM_Q : DV_T);
+    dp.ktiles = (int)ceil_div(D.M, mfma ? DM_K : DV_T);
+    const unsigned grid = (unsigned)(8 * ceil_div((int64_t)dp.qtiles * dp.ktiles * dp.nbh, 8));
+    if constexpr (!std::is_same<T, float>::value) {
+        if (mfma) {
+#define SSA_DENSE(DD) \
+    case DD: hipLaunchKernelGGL((dense_mfma_kernel<T, DD>), dim3(grid), dim3(256), 0, st, dp); break;
+            switch (mfma_instance(D.d)) {
+                SSA_DENSE(8) SSA_DENSE(16) SSA_DENSE(32) SSA_DENSE(64) SSA_DENSE(96) SSA_DENSE(128)
+                default: ssa_set_error("dense scores: head dim %d", D.d); return SSA_E_UNSUP;
+            }
+#undef SSA_DENSE
+            SSA_CHECK_LAUNCH();
+            return SSA_OK;
+        }
+    }
+    hipLaunchKernelGGL((dense_valu_kernel<T>), dim3(grid), dim3(256), 0, st, dp);
+    SSA_CHECK_LAUNCH();
+    return SSA_OK;
+}
+
+template <typename T, bool CAUSAL>
+int dense_select_c(const SelP &sp0, hipStream_t st) {
+    SelP sp = sp0;
+    sp.waves = SEL_WAVES;
+    sp.nblocks = ceil_div(sp.rows, SEL_WAVES);
+    const dim3 grid((unsigned)(8 * ceil_div(sp.nblocks, 8))), block(SEL_WAVES * SSA_WAVE);
+    const int blocks = (int)ceil_div(sp.M, DN_BLK);
+    if (blocks <= 4) hipLaunchKernelGGL((select_dense_kernel<T, CAUSAL, 4>), grid, block, 0, st, sp);
+    else if (blocks <= 8) hipLaunchKernelGGL((select_dense_kernel<T, CAUSAL, 8>), grid, block, 0, st, sp);
+    else if (blocks <= 16) hipLaunchKernelGGL((select_dense_kernel<T, CAUSAL, 16>), grid, block, 0, st, sp);
+    else hipLaunchKernelGGL((select_dense_kernel<T, CAUSAL, 32>), grid, block, 0, st, sp);
+    SSA_CHECK_LAUNCH();
+    return SSA_OK;
+}
+
+template <typename T>
+int dense_select(const SelP &sp, hipStream_t st) {
+    return sp.causal ? dense_select_c<T, true>(sp, st) : dense_select_c<T, false>(sp, st);
+}
+
 // Query phase: everything else, given the key phase's results in ws.
 template <typename T>
 int queries_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws,
@@ -4313,8 +4466,20 @@ int queries_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char 
         // writes, and the query buckets need the ids it writes when fused
         // (the first chunk's ran beside the key sort when sort_aux)
         const AuxP ap = aux_params(D, a, L, ws, bh0, nbh, fuse_qhash);
-        if (!D.fused && !(sort_aux && bh0 == 0)) rc = aux_dispatch<T>(D.d, mfma, ap, st);
+        // (dense without the matrix cores: the score kernel takes the scales)
+        if (!D.fused && !(sort_aux && bh0 == 0) && (mfma || !D.dense))
+            rc = aux_dispatch<T>(D.d, mfma, ap, st);
         if (rc) return rc;
+        if (D.dense) {
+            SelP sp = select_common<T>(D, a, L, ws, bh0, nbh, mfma);
+            sp.aux = mfma ? ap.out : nullptr;
+            sp.NA = ap.NA;
+            rc = dense_scores<T>(D, a, L, ws, sp, st);
+            if (!rc) rc = dense_select<T>(sp, st);
+            if (rc) return rc;
+            last = sp;
+            continue;
+        }
         QbP qp = qb_params(D, a, L, ws, bh0, nbh);
         const dim3 gq((unsigned)ceil_div(D.N, 256), (unsigned)ninst);
         // (the first chunk's histogram and scan ran in the key phase when sort_aux)
@@ -4357,32 +4522,13 @@ int queries_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char 
         rc = rescore_dispatch<T>(D.d, rp, grid, st);
         if (rc) return rc;
 
-        SelP sp{};
-        sp.qid = qp.qid; sp.perm = cp.perm; sp.bstart = rp.bstart; sp.bsize = rp.bsize;
+        SelP sp = select_common<T>(D, a, L, ws, bh0, nbh, mfma);
         sp.sid = rp.sid; sp.rnk = (const int32_t *)(ws + L.rnk);
         sp.inv = (const int32_t *)(ws + L.inv); sp.cut = cp.cut; sp.srix = cp.srix;
         sp.head_bytes = (uint32_t)((int64_t)D.N * D.nlists * D.Cs * 2);
-        sp.mfma = mfma ? 1 : 0;
-        sp.nl_magic = (uint32_t)((((uint64_t)1 << 32) + D.nlists - 1) / D.nlists);
-        sp.S = rp.S; sp.q = a->q.ptr; sp.k = a->k.ptr;
-        sp.qsb = a->q.sb; sp.qsh = a->q.sh; sp.qsn = a->q.sn;
-        sp.ksb = a->k.sb; sp.ksh = a->k.sh; sp.ksn = a->k.sn;
-        sp.glob = a->glob;
-        sp.N = D.N; sp.M = D.M; sp.d = D.d; sp.R = D.R; sp.NS = D.NS; sp.NB = D.NB; sp.C = D.C;
-        sp.Cs = D.Cs;
-        sp.CPL = D.CPL; sp.nlists = D.nlists; sp.Hq = D.Hq; sp.Hkv = D.Hkv; sp.rep = D.rep;
-        sp.G = D.G; sp.kk = D.kk; sp.window = a->window; sp.causal = a->causal;
-        sp.cross = a->is_cross; sp.mode = a->mode; sp.total_k = a->total_k; sp.Kw = D.Kw;
-        sp.Kout = D.Kout; sp.bh0 = (int)bh0; sp.words = sel_bitmap_words(D.M);
-        sp.Call = D.Call; sp.rows = (int64_t)nbh * D.N; sp.rows_all = D.BH * D.N;
-        sp.out_idx = a->out_idx; sp.out_valid = a->out_valid; sp.ties = a->out_ties;
-        sp.out_idx32 = a->mode == SSA_GRAPH_FULL ? a->out_idx32 : nullptr;
-        sp.tie_list = (int32_t *)(ws + L.tie_list);
-        sp.tie_count = (int32_t *)(ws + L.tie_count);
+        sp.S = rp.S;
         sp.aux = ap.out;
         sp.NA = ap.NA;
-        sp.perm_bytes = (int)(D.BK * D.R * D.M * 4);
-        sp.cbits = D.cbits;
         rc = select_dispatch<T>(sp, st);
         if (rc) return rc;
         last = sp;
