@@ -12,9 +12,9 @@
 //                          rows in LDS; the count before a slot is its rank
 //                          (48 us)
 //   2. grad_chunk_kernel,  prefixes over the blocks and over the key rows: the
-//      grad_list_kernel    place of every slot in its key row's list, and the
-//                          lists cut into segments of at most `seg` entries
-//                          (15 + 43 us)
+//      grad_list_kernel,   place of every slot in its key row's list, and the
+//      grad_segs_kernel    lists cut into segments of at most `seg` entries
+//                          (15 + 8 + 5 us)
 //   3. grad_rows_kernel    per query row: scores and dO.V, the softmax, dQ;
 //                          each slot's two weights go to its place in the list
 //                          (772 us)
@@ -64,6 +64,7 @@ struct GradP {
     uint32_t *tab;         // (ng, nc, M) slots before this block
     int64_t *kbegin;       // (ng, M)
     uint32_t *klen;        // (ng, M)
+    int32_t *kfirst;       // (ng, M) first segment
     int2 *kpart;           // (ng, M) first partial, partials (0: none)
     uint32_t *wmax;        // (ng, M, 2) largest |draw|, |p'| as float bits (deterministic)
     uint8_t *poison;       // (ng, M) 1: dK is NaN, 2: dV is NaN
@@ -145,50 +146,78 @@ __device__ __forceinline__ V wave_scan_incl(V v, int lane) {
     return v;
 }
 
-// one workgroup per group: where each key row's list starts, and its segments
+// One workgroup per group: where each key row's list, segments and partials
+// start.  A thread sums LIST_KEYS consecutive key rows, so a group of up to
+// 8,192 takes one round of scans.
+constexpr int LIST_KEYS = 8;
 __global__ void __launch_bounds__(1024) grad_list_kernel(GradP p) {
     __shared__ int64_t wl[16];
     __shared__ int32_t ws[16], wp[16];
     const int gl = blockIdx.x, tid = threadIdx.x, lane = lane_id(), wid = tid / SSA_WAVE;
     int64_t cl = (int64_t)gl * p.gslots;        // entries before this tile
     int32_t cs = 0, cp = 0;                     // segments, partials before it
-    for (int k0 = 0; k0 < p.a.M; k0 += 1024) {
-        const int x = k0 + tid;
-        const int64_t i = (int64_t)gl * p.a.M + x;
-        const uint32_t len = x < p.a.M ? p.klen[i] : 0u;
-        const int ns = x < p.a.M ? (len ? (int)((len + p.seg - 1) / p.seg) : 1) : 0;
-        const int np = ns > 1 ? ns : 0;
-        const int64_t il = wave_scan_incl<int64_t>((int64_t)len, lane);
-        const int is = wave_scan_incl<int>(ns, lane), ip = wave_scan_incl<int>(np, lane);
+    for (int k0 = 0; k0 < p.a.M; k0 += 1024 * LIST_KEYS) {
+        const int x0 = k0 + tid * LIST_KEYS;
+        const int64_t i0 = (int64_t)gl * p.a.M + x0;
+        uint32_t len[LIST_KEYS];
+        int64_t tl = 0;
+        int ts = 0, tp = 0;
+#pragma unroll
+        for (int u = 0; u < LIST_KEYS; ++u) len[u] = x0 + u < p.a.M ? p.klen[i0 + u] : 0u;
+#pragma unroll
+        for (int u = 0; u < LIST_KEYS; ++u) {
+            const int ns = x0 + u < p.a.M ? (len[u] ? (int)((len[u] + p.seg - 1) / p.seg) : 1) : 0;
+            tl += len[u];
+            ts += ns;
+            tp += ns > 1 ? ns : 0;
+        }
+        const int64_t il = wave_scan_incl<int64_t>(tl, lane);
+        const int is = wave_scan_incl<int>(ts, lane), ip = wave_scan_incl<int>(tp, lane);
         if (lane == SSA_WAVE - 1) { wl[wid] = il; ws[wid] = is; wp[wid] = ip; }
         __syncthreads();
-        int64_t bl = 0, tl = 0;
-        int bs = 0, ts = 0, bp = 0, tp = 0;
+        int64_t bl = cl + il - tl, al = 0;
+        int bs = cs + is - ts, as = 0, bp = cp + ip - tp, ap = 0;
         for (int w = 0; w < 16; ++w) {
             if (w < wid) { bl += wl[w]; bs += ws[w]; bp += wp[w]; }
-            tl += wl[w]; ts += ws[w]; tp += wp[w];
+            al += wl[w]; as += ws[w]; ap += wp[w];
         }
-        if (x < p.a.M) {
-            const int64_t begin = cl + bl + il - len;
-            const int s0 = cs + bs + is - ns;
-            const int p0 = np ? (int)((int64_t)gl * p.partcap) + cp + bp + ip - np : -1;
-            p.kbegin[i] = begin;
-            p.kpart[i] = make_int2(p0, np);
-            for (int s = 0; s < ns; ++s) {
-                GradSeg d;
-                d.begin = begin + (int64_t)s * p.seg;
-                const int64_t left = (int64_t)len - (int64_t)s * p.seg;
-                d.len = (int)(left < p.seg ? left : p.seg);
-                d.key = x;
-                d.part = np ? p0 + s : -1;
-                d.pad = 0;
-                p.segs[(int64_t)gl * p.segcap + s0 + s] = d;
+#pragma unroll
+        for (int u = 0; u < LIST_KEYS; ++u) {
+            if (x0 + u < p.a.M) {
+                const int ns = len[u] ? (int)((len[u] + p.seg - 1) / p.seg) : 1;
+                const int np = ns > 1 ? ns : 0;
+                p.kbegin[i0 + u] = bl;
+                p.kfirst[i0 + u] = bs;
+                p.kpart[i0 + u] = make_int2(np ? (int)((int64_t)gl * p.partcap) + bp : -1, np);
+                bl += len[u]; bs += ns; bp += np;
             }
         }
-        cl += tl; cs += ts; cp += tp;
+        cl += al; cs += as; cp += ap;
         __syncthreads();
     }
     if (tid == 0) p.nseg[gl] = cs;
+}
+
+// thread per (group, key row): its segments
+__global__ void __launch_bounds__(256) grad_segs_kernel(GradP p) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)p.ng * p.a.M) return;
+    const int64_t gl = i / p.a.M;
+    const uint32_t len = p.klen[i];
+    const int2 kp = p.kpart[i];
+    const int ns = kp.y ? kp.y : 1;
+    const int64_t begin = p.kbegin[i];
+    GradSeg *out = p.segs + gl * p.segcap + p.kfirst[i];
+    for (int s = 0; s < ns; ++s) {
+        GradSeg d;
+        d.begin = begin + (int64_t)s * p.seg;
+        const int64_t left = (int64_t)len - (int64_t)s * p.seg;
+        d.len = (int)(left < p.seg ? left : p.seg);
+        d.key = (int)(i - gl * p.a.M);
+        d.part = kp.y ? kp.x + s : -1;
+        d.pad = 0;
+        out[s] = d;
+    }
 }
 
 // ---------------------------------------------------------------- 3. query rows
@@ -831,20 +860,41 @@ __global__ void __launch_bounds__(WAVES * SSA_WAVE) grad_join_kernel(GradP gp) {
     }
 }
 
-// largest |x| over a (B, H, N, d) view, as float bits (deterministic mode)
-template <typename T>
-__global__ void __launch_bounds__(256) grad_absmax_kernel(const T *x, int64_t sb, int64_t sh,
-                                                          int64_t sn, int H, int N, int d,
-                                                          int64_t rows, uint32_t *out) {
+// Largest |x| over the rows of a (B, H, N, d) view, as float bits
+// (deterministic mode): a lane group per row, a row's elements in pieces of
+// VEC, one atomic per workgroup.
+template <typename T, int D>
+__device__ __forceinline__ uint32_t rows_absmax(const T *x, int64_t sb, int64_t sh, int64_t sn, int H,
+                                                int N, int d, int64_t rows) {
+    using G = Geo<T, D>;
+    constexpr int VEC = G::VEC, LPR = G::LPR, RPB = 256 / LPR;
+    const int li = threadIdx.x % LPR;
     uint32_t m = 0;
-    const int64_t total = rows * d;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-        const int64_t r = i / d, e = i % d;
-        const int64_t n = r % N, bh = r / N;
-        m = max(m, abs_bits(to_f32(x[(bh / H) * sb + (bh % H) * sh + n * sn + e])));
+    if (li * VEC < d) {
+        for (int64_t r = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR; r < rows;
+             r += (int64_t)gridDim.x * RPB) {
+            const uint32_t bh = (uint32_t)(r / N);
+            const Raw<T, VEC> v = load_raw<T, VEC>(x + (int64_t)(bh / (uint32_t)H) * sb +
+                                                   (int64_t)(bh % (uint32_t)H) * sh + (r - (int64_t)bh * N) * sn +
+                                                   li * VEC);
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) m = max(m, abs_bits(to_f32(v.e[e])));
+        }
     }
-    m = wave_max_u(m);
-    if (lane_id() == 0) atomicMax(out, m);
+    return wave_max_u(m);
+}
+
+// workgroups alternate between q (xmax[0]) and dO (xmax[1])
+template <typename T, typename TD, int D>
+__global__ void __launch_bounds__(256) grad_absmax_kernel(GradP p) {
+    __shared__ uint32_t red[4];
+    const ApplyP &a = p.a;
+    const uint32_t m = blockIdx.y == 0
+        ? rows_absmax<T, D>((const T *)a.q, a.qsb, a.qsh, a.qsn, a.Hq, a.N, a.d, a.rows)
+        : rows_absmax<TD, D>((const TD *)p.dout, p.dosb, p.dosh, p.dosn, a.Hq, a.N, a.d, a.rows);
+    if (lane_id() == 0) red[threadIdx.x / SSA_WAVE] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(&p.xmax[blockIdx.y], max(max(red[0], red[1]), max(red[2], red[3])));
 }
 
 __global__ void __launch_bounds__(256) grad_zero_kernel(uint32_t *w, int64_t n) {
@@ -870,7 +920,7 @@ constexpr int64_t GRAD_SLOTS = (int64_t)1 << 28;   // slots per launch: 5.4 GB o
 int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
 struct GradLayout {
-    int64_t ent, rank, tab, kbegin, klen, kpart, wmax, poison, segs, nseg, part, xmax, total;
+    int64_t ent, rank, tab, kbegin, klen, kfirst, kpart, wmax, poison, segs, nseg, part, xmax, total;
 };
 
 // Sizes of one launch over `ng` groups (whole (b, kv head) groups, so no key
@@ -897,6 +947,7 @@ GradLayout grad_plan(GradP &p, int det) {
     L.tab = take((int64_t)p.ng * p.nc * p.a.M * 4);
     L.kbegin = take(keys * 8);
     L.klen = take(keys * 4);
+    L.kfirst = take(keys * 4);
     L.kpart = take(keys * 8);
     L.wmax = take(det ? keys * 8 : 0);
     L.poison = take(keys + 4);
@@ -947,6 +998,7 @@ int launch_grad(GradP p, int det, char *ws, hipStream_t st) {
     p.tab = (uint32_t *)(ws + L.tab);
     p.kbegin = (int64_t *)(ws + L.kbegin);
     p.klen = (uint32_t *)(ws + L.klen);
+    p.kfirst = (int32_t *)(ws + L.kfirst);
     p.kpart = (int2 *)(ws + L.kpart);
     p.wmax = det ? (uint32_t *)(ws + L.wmax) : nullptr;
     p.poison = (uint8_t *)(ws + L.poison);
@@ -958,13 +1010,8 @@ int launch_grad(GradP p, int det, char *ws, hipStream_t st) {
     if (det) {
         hipLaunchKernelGGL(grad_zero_kernel, dim3(1), dim3(256), 0, st, p.xmax, (int64_t)2);
         SSA_CHECK_LAUNCH();
-        const int64_t rows = (int64_t)a.B * a.Hq * a.N;
-        const unsigned gr = (unsigned)std::min<int64_t>(ceil_div(rows * a.d, 2048), 1024);
-        hipLaunchKernelGGL((grad_absmax_kernel<T>), dim3(gr), dim3(256), 0, st, (const T *)a.q, a.qsb,
-                           a.qsh, a.qsn, a.Hq, a.N, a.d, rows, p.xmax);
-        SSA_CHECK_LAUNCH();
-        hipLaunchKernelGGL((grad_absmax_kernel<TD>), dim3(gr), dim3(256), 0, st, (const TD *)p.dout,
-                           p.dosb, p.dosh, p.dosn, a.Hq, a.N, a.d, rows, p.xmax + 1);
+        const unsigned gr = (unsigned)std::min<int64_t>(ceil_div(a.rows, 256), 256);
+        hipLaunchKernelGGL((grad_absmax_kernel<T, TD, D>), dim3(gr, 2), dim3(256), 0, st, p);
         SSA_CHECK_LAUNCH();
     }
     const size_t clds = (size_t)std::min(a.M, CNT_KEYS) * 4;
@@ -978,6 +1025,8 @@ int launch_grad(GradP p, int det, char *ws, hipStream_t st) {
         hipLaunchKernelGGL(grad_chunk_kernel, dim3((unsigned)ceil_div(keys, 256)), dim3(256), 0, st, p);
         SSA_CHECK_LAUNCH();
         hipLaunchKernelGGL(grad_list_kernel, dim3((unsigned)p.ng), dim3(1024), 0, st, p);
+        SSA_CHECK_LAUNCH();
+        hipLaunchKernelGGL(grad_segs_kernel, dim3((unsigned)ceil_div(keys, 256)), dim3(256), 0, st, p);
         SSA_CHECK_LAUNCH();
         const unsigned grid = (unsigned)(8 * ceil_div(ceil_div((int64_t)p.ng * p.grows, WAVES), 8));
         if (a.K > GRAD_KLDS) {
