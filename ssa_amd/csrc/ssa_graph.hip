@@ -3596,13 +3596,22 @@ Layout plan(const Dims &D) {
 
 // Whether the build takes the dense form (ssa_graph_dense.h): a graph, keys
 // within a select row's registers, lists within a wave's lanes, a round's
-// bitmaps within LDS, and lists that hold in all at least as many members as
-// there are keys (below that the list form reads fewer scores).
+// bitmaps within LDS, and enough list members (over a row's lists) per key.
+// Where that line lies was measured with both forms (whole build, list / dense
+// us): 16-bit rows, 4,096 causal keys, d = 64: 0.9 members per key 413 / 436,
+// 1.8: 753 / 621; 2,048 keys: 0.8: 188 / 187, 1.8: 234 / 191; 1,024 keys: 0.25:
+// 177 / 164, 0.8: 156 / 136; 512 keys (cross): 0.5: 223 / 187.  fp32, whose list
+// rescore runs on the vector units: 4,096 keys: 0.2: 384 / 553 (cross) and 520 /
+// 602 (causal), 0.4: 535 / 550 and 836 / 731; 2,048 keys: 0.4: 352 / 322 and 324 /
+// 251; 1,024 keys: 0.25: 293 / 200.
 bool dense_form(const Dims &D, const ssa_graph_args *a) {
     const int64_t nw = ceil_div(D.M, 64);
+    if (a->mode != SSA_GRAPH_FULL || D.M > DN_MAX_KEYS || D.nlists > DN_MAX_LISTS ||
+        D.NB * (nw * 8 + 4) > DN_BITS_LDS)
+        return false;
     const int64_t members = (int64_t)D.nlists * std::min<int64_t>(D.C, ceil_div(D.M, D.NB));
-    return a->mode == SSA_GRAPH_FULL && D.M <= DN_MAX_KEYS && D.nlists <= DN_MAX_LISTS &&
-           D.NB * (nw * 8 + 4) <= DN_BITS_LDS && members * DN_NUM >= D.M * (int64_t)DN_DEN;
+    if (D.M <= 1024) return members * 4 >= D.M;
+    return a->q.dtype == SSA_F32 ? members * 5 >= (int64_t)D.M * 2 : members >= D.M;
 }
 
 Layout plan(const Dims &D);

@@ -22,7 +22,6 @@ constexpr int DN_BLK = 128;            // keys per block of a score row
 constexpr int DN_MAX_KEYS = 4096;      // keys a select row holds in registers
 constexpr int DN_MAX_LISTS = 64;       // one lane per list
 constexpr int DN_BITS_LDS = 65536;     // bytes of one round's bitmaps
-constexpr int DN_NUM = 1, DN_DEN = 1;  // dense where list members x DN_NUM >= keys x DN_DEN
 
 // Score row of a query: Ms codes (M rounded up to DN_BLK, one block more where
 // that is a multiple of 1,024 codes: rows a multiple of 2 KB apart would share
@@ -96,16 +95,20 @@ __global__ void __launch_bounds__(1024) list_bits_kernel(LbP p) {
 }
 
 // ---------------------------------------------------------------- scores
-constexpr int DM_Q = 128;              // queries per workgroup: 32 per wave
+constexpr int DM_QF = 4;               // 16-query operands per wave
+constexpr int DM_Q = 64 * DM_QF;       // queries per workgroup
 constexpr int DM_K = 512;              // keys per workgroup: 4 blocks
 
 // 16-bit q and k on the matrix cores, with the k steps, operand roles and so
-// the sums of the list form's rescore.  A wave holds 32 queries as B operands
+// the sums of the list form's rescore.  A wave holds 64 queries as B operands
 // and walks its keys in pairs of 16-row tiles 64 keys apart, whose results are
 // the four 32-bit pairs a lane stores with one 16-byte store; the next pair's K
 // rows load while this one multiplies.  K rows come straight from the L1 (the
-// four waves walk the same rows).  Bound: the code stores (0.54 GB at 32 heads
-// of 4,096 causal queries).
+// four waves walk the same rows).  Loads and stores of a wave retire in order,
+// so a load issued behind a store waits for it: a block's stores go out together
+// behind the next block's first loads.  Bound: the K fragments' way through the
+// L1 (64 queries a wave instead of 32, which halves them: 95 -> 72 us at 16 heads
+// of 2,999 causal rows, d = 96; 0.14 GB of codes).
 template <typename T, int D>
 __global__ void __launch_bounds__(256) dense_mfma_kernel(DnP p) {
     using V = typename Mfma16<T>::vec;
@@ -117,21 +120,21 @@ __global__ void __launch_bounds__(256) dense_mfma_kernel(DnP p) {
     const int t = (int)(blk % tiles);
     const int qt = t / p.ktiles, kt = t % p.ktiles;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / SSA_WAVE);
-    const int n0 = qt * DM_Q + 32 * wid;
+    const int n0 = qt * DM_Q + 16 * DM_QF * wid;
     const int k0 = kt * DM_K;
     // causal: keys up to the wave's last query
     int kend = min(k0 + DM_K, (p.M + DN_BLK - 1) / DN_BLK * DN_BLK);
-    if (p.causal) kend = min(kend, (min(n0 + 31, p.N - 1) / DN_BLK + 1) * DN_BLK);
+    if (p.causal) kend = min(kend, (min(n0 + 16 * DM_QF - 1, p.N - 1) / DN_BLK + 1) * DN_BLK);
     if (n0 >= p.N || k0 >= kend) return;
     const int bh = p.bh0 + bhl, b = bh / p.Hq, h = bh % p.Hq, g = h / p.rep;
     const int lane = lane_id(), li = lane % 16, lg = lane / 16;
     const T *qbase = (const T *)p.q + b * p.qsb + h * p.qsh;
     const T *kbase = (const T *)p.k + b * p.ksb + g * p.ksh;
     const V zero = __builtin_bit_cast(V, make_uint4(0, 0, 0, 0));
-    V qf[2][KS];
-    float sc[2];
+    V qf[DM_QF][KS];
+    float sc[DM_QF];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < DM_QF; ++i) {
         const int n = min(n0 + 16 * i + li, p.N - 1);
         sc[i] = p.aux[((int64_t)bhl * p.N + n) * p.NA + p.NA - 1];
 #pragma unroll
@@ -153,39 +156,40 @@ __global__ void __launch_bounds__(256) dense_mfma_kernel(DnP p) {
             }
         }
     };
-    uint32_t *srow = p.S + ((int64_t)bhl * p.N + n0 + li) * (p.Ms / 2);
-    auto score = [&](int x, const V (&a)[2][KS]) __attribute__((always_inline)) {
+    uint32_t *srow = p.S + ((int64_t)bhl * p.N + n0 + li) * (p.Ms / 2) + 4 * lg;
+    uint4 w[4][DM_QF];                     // the block's codes: tile pair, 16 queries
+    auto score = [&](const V (&a)[2][KS], uint4 (&o)[DM_QF]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < DM_QF; ++i) {
             f32x4_t c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0;
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
                 c0 = Mfma16<T>::mma(a[0][s], qf[i][s], c0);
                 c1 = Mfma16<T>::mma(a[1][s], qf[i][s], c1);
             }
-            // lane (li, lg): keys x + 4 lg + r (and + 64) for query n0 + 16 i + li
-            uint4 w;
-            w.x = dn_pair(c0[0], c1[0], sc[i]);
-            w.y = dn_pair(c0[1], c1[1], sc[i]);
-            w.z = dn_pair(c0[2], c1[2], sc[i]);
-            w.w = dn_pair(c0[3], c1[3], sc[i]);
-            const int blk128 = x / DN_BLK, off = x % DN_BLK;
-            if (n0 + 16 * i + li < p.N)
-                *reinterpret_cast<uint4 *>(srow + (int64_t)16 * i * (p.Ms / 2) + 64 * blk128 + off + 4 * lg) = w;
+            // lane (li, lg): keys 4 lg + r (and 64 on) of the pair for query n0 + 16 i + li
+            o[i] = make_uint4(dn_pair(c0[0], c1[0], sc[i]), dn_pair(c0[1], c1[1], sc[i]),
+                              dn_pair(c0[2], c1[2], sc[i]), dn_pair(c0[3], c1[3], sc[i]));
         }
     };
-    // keys x = 128 b + 16 a, a = 0..3
-    auto next = [](int x) { return (x & 48) == 48 ? x + 80 : x + 16; };
     V a0[2][KS], a1[2][KS];
     load(k0, a0);
-    for (int x = k0; x < kend;) {
-        const int y = next(x);
-        load(y < kend ? y : x, a1);
-        score(x, a0);
-        if (y >= kend) break;
-        x = next(y);
-        load(x < kend ? x : y, a0);
-        score(y, a1);
+    for (int x = k0; x < kend; x += DN_BLK) {
+        load(x + 16, a1);
+        score(a0, w[0]);
+        load(x + 32, a0);
+        score(a1, w[1]);
+        load(x + 48, a1);
+        score(a0, w[2]);
+        // the next block's first rows before this block's stores
+        load(min(x + DN_BLK, kend - DN_BLK), a0);
+        score(a1, w[3]);
+#pragma unroll
+        for (int i = 0; i < DM_QF; ++i)
+            if (n0 + 16 * i + li < p.N)
+#pragma unroll
+                for (int a = 0; a < 4; ++a)
+                    *reinterpret_cast<uint4 *>(srow + (int64_t)16 * i * (p.Ms / 2) + x / 2 + 16 * a) = w[a][i];
     }
 }
 
@@ -598,22 +602,22 @@ __global__ void __launch_bounds__(SEL_WAVES * SSA_WAVE) select_dense_kernel(SelP
                 if (lane == 2 * b) eq = e0;
                 if (lane == 2 * b + 1) eq = e1;
             });
-            const int ne = clo - chi;
             const int elo = (int)(uint32_t)eq, ehi = (int)(uint32_t)(eq >> 32);
             auto echunk = [&](int c) {
                 return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(ehi, c) << 32) |
                        (uint32_t)__builtin_amdgcn_readlane(elo, c);
             };
             uint64_t nz = wave_ballot(eq != 0ull);
-            if (ne <= DN_CAP) {
+            if (clo - chi <= DN_CAP) {
                 // their exact keys in LDS decide
                 uint32_t *ids = scr, *keys = scr + DN_CAP;
-                int at = 0;
+                int ne = 0;
                 for (uint64_t z = nz; z; z &= z - 1ull) {
                     const int c = __ffsll((long long)z) - 1;
                     const uint64_t m = echunk(c);
-                    if (in_mask(m)) ids[at + lanes_below(m)] = (uint32_t)(64 * c + lane);
-                    at += __popcll(m);
+                    const int at = ne + lanes_below(m);
+                    if (in_mask(m) && at < DN_CAP) ids[at] = (uint32_t)(64 * c + lane);
+                    ne = min(ne + __popcll(m), DN_CAP);
                 }
                 wave_lds_sync();
                 uint32_t kv[DN_CAP / SSA_WAVE];
