@@ -195,7 +195,15 @@ def require_device(*tensors):
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """Handle of the current stream of t's device (the raw query: building a
+    torch.cuda.Stream object for it takes 5 us of a small call)."""
+    i = t.device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if i is None else i)
+
+
+def _plain(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """t as a contiguous tensor of dtype, t itself where it is one."""
+    return t if t.dtype == dtype and t.is_contiguous() else t.detach().to(dtype).contiguous()
 
 
 def dtype_code(dt: torch.dtype) -> int:
@@ -259,8 +267,8 @@ def _graph_args(q, k, rand_proj, *, P, T, C, top_k, window, causal, is_cross, to
         raise RuntimeError("ssa_amd.build_graph: q and k dtypes differ")
     qa, qk = view4(q)
     ka, kk_ = view4(k)
-    rp = rand_proj.detach().to(torch.float32).contiguous()
-    g = glob.detach().to(device=q.device, dtype=torch.int64).contiguous()
+    rp = _plain(rand_proj, torch.float32)
+    g = _plain(glob if glob.device == q.device else glob.detach().to(q.device), torch.int64)
     qp = q_proj.detach().to(torch.float32).contiguous() if q_proj is not None else None
     kp = k_proj.detach().to(torch.float32).contiguous() if k_proj is not None else None
     a = GraphArgs()
@@ -515,8 +523,8 @@ def check_apply_shapes(q, k, v, neighbors, valid, out=None):
 
 def _apply_args(q, k, v, neighbors, valid, scale, fp32w, dropout_p, seed, out, ids32=True):
     """int32 neighbours without a mask are passed as they are (a negative id
-    is an invalid slot, as the int64 path treats it) when ids32 allows."""
-    check_apply_shapes(q, k, v, neighbors, valid, out)
+    is an invalid slot, as the int64 path treats it) when ids32 allows.  The
+    caller has checked the operands' shapes."""
     B, Hq, N, d = q.shape
     _, Hkv, M, _ = k.shape
     K = neighbors.shape[-1]
@@ -540,12 +548,15 @@ def _apply_args(q, k, v, neighbors, valid, scale, fp32w, dropout_p, seed, out, i
 
 
 def gather_attention_fwd(q, k, v, neighbors, valid, scale, fp32w=False, dropout_p=0.0, seed=0,
-                         out=None, row_invalid=None):
+                         out=None, row_invalid=None, *, _checked=False):
     """row_invalid: optional (B*Hq*N,) int32, written with each query row's
     count of slots the graph marks invalid (valid false, or a negative int32
-    id): the reference's padding statistic."""
-    check_apply_shapes(q, k, v, neighbors, valid, out)
-    require_device(q, k, v, neighbors, valid, row_invalid)
+    id): the reference's padding statistic.  _checked: the caller has checked
+    shapes and devices (no out given)."""
+    if not _checked:
+        check_apply_shapes(q, k, v, neighbors, valid, out)
+        require_device(q, k, v, neighbors, valid)
+    require_device(row_invalid)
     if row_invalid is not None:
         B, Hq, N, _ = q.shape
         if (row_invalid.dtype != torch.int32 or row_invalid.numel() != B * Hq * N

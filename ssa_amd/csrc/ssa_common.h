@@ -34,6 +34,17 @@ void ssa_set_error(const char *fmt, ...);
 
 #define SSA_CHECK_LAUNCH() SSA_CHECK_HIP(hipGetLastError())
 
+// Raises kernel fn's limit of dynamic LDS to `bytes` where the default could be
+// too low (64 KB with the kernel's static LDS, below 32 KB in every kernel
+// here); most launches need no call.
+#define SSA_ALLOW_LDS(fn, bytes)                                                               \
+    do {                                                                                       \
+        if ((size_t)(bytes) > 32768)                                                           \
+            SSA_CHECK_HIP(hipFuncSetAttribute((const void *)(fn),                              \
+                                              hipFuncAttributeMaxDynamicSharedMemorySize,      \
+                                              (int)(bytes)));                                  \
+    } while (0)
+
 // ---------------------------------------------------------------- dtypes
 // 16-bit storage types as raw bits: bf16 = upper half of an fp32, fp16 = IEEE
 // binary16.  Conversions are written out so the numerics are explicit.

@@ -44,6 +44,7 @@
 #include <stdio.h>
 
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #include "ssa_common.h"
@@ -125,8 +126,8 @@ struct HashP {
     uint32_t *kpart;    // key hash: max |k|^2 of each 16-row tile as float bits, or null
 };
 
-__device__ __forceinline__ void hash_clear(const HashP &p) {
-    if (blockIdx.x == 0) {
+__device__ __forceinline__ void hash_clear(const HashP &p, int blk) {
+    if (blk == 0) {
         for (int i = threadIdx.x; i < p.nzero; i += blockDim.x) p.zero[i] = 0u;
         if (p.zero1 && threadIdx.x == 0) *p.zero1 = 0;
     }
@@ -134,7 +135,7 @@ __device__ __forceinline__ void hash_clear(const HashP &p) {
 
 template <typename T>
 __global__ void __launch_bounds__(256) hash_kernel(HashP p) {
-    hash_clear(p);
+    hash_clear(p, (int)blockIdx.x);
     const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (row >= p.rows) return;
     const int i = (int)(row % p.L);
@@ -204,7 +205,7 @@ __global__ void __launch_bounds__(256) hash_kernel(HashP p) {
 // instance's head dim; the rows' own d <= D: elements past d are zero in the
 // rows and the planes.
 template <typename T, int D>
-__global__ void __launch_bounds__(256) hash_mfma_kernel(HashP p) {
+__device__ void hash_mfma_block(const HashP &p, int blk) {
     constexpr int DQ = D / 4;
     constexpr int CH = DQ < 32 ? DQ : 32;             // plane elements loaded per group
     extern __shared__ float hs[];
@@ -212,13 +213,13 @@ __global__ void __launch_bounds__(256) hash_mfma_kernel(HashP p) {
     const int NT = (NP + 15) / 16;
     float *proj = hs;                                 // [4 waves][16][NT*16 + 1]
     const int pst = NT * 16 + 1;
-    hash_clear(p);
+    hash_clear(p, blk);
     const int wid = threadIdx.x / SSA_WAVE;
     const int lane = lane_id();
     const int li = lane % 16, lg = lane / 16;
     {
         // the block's 4 waves take adjacent 16-row tiles
-        const int64_t row0 = ((int64_t)blockIdx.x * 4 + wid) * 16;
+        const int64_t row0 = ((int64_t)blk * 4 + wid) * 16;
         if (row0 >= p.rows) return;
         const int64_t row = row0 + li;
         float xs[DQ];
@@ -330,6 +331,18 @@ __global__ void __launch_bounds__(256) hash_mfma_kernel(HashP p) {
             }
         }
     }
+}
+
+template <typename T, int D>
+__global__ void __launch_bounds__(256) hash_mfma_kernel(HashP p) {
+    hash_mfma_block<T, D>(p, (int)blockIdx.x);
+}
+
+// keys (the first kblocks workgroups) and queries in one launch
+template <typename T, int D>
+__global__ void __launch_bounds__(256) hash_mfma2_kernel(HashP k, HashP q, int kblocks) {
+    if ((int)blockIdx.x < kblocks) hash_mfma_block<T, D>(k, (int)blockIdx.x);
+    else hash_mfma_block<T, D>(q, (int)blockIdx.x - kblocks);
 }
 
 // ------------------------------------------------------------------ small utilities
@@ -3794,24 +3807,31 @@ int make_dims(const ssa_graph_args *a, Dims &D, bool need_q = true, int64_t ws_c
     return SSA_OK;
 }
 
+// hash of hp's rows, and of also's (same planes) when given
 template <typename T, int Dh>
-int launch_hash_mfma(const HashP &hp, hipStream_t st) {
+int launch_hash_mfma(const HashP &hp, const HashP *also, hipStream_t st) {
     const int NT = (hp.R * hp.P + 15) / 16;
     const size_t lds = (size_t)4 * 16 * (NT * 16 + 1) * 4;
     if (lds > SSA_LDS_BYTES) {
         ssa_set_error("hash: %d planes need %zu bytes of LDS", hp.R * hp.P, lds);
         return SSA_E_UNSUP;
     }
-    SSA_CHECK_HIP(hipFuncSetAttribute((const void *)hash_mfma_kernel<T, Dh>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((hash_mfma_kernel<T, Dh>), dim3((unsigned)ceil_div(hp.rows, 64)), dim3(256),
-                       lds, st, hp);
+    const int64_t nb = ceil_div(hp.rows, 64);
+    if (also) {
+        SSA_ALLOW_LDS((hash_mfma2_kernel<T, Dh>), lds);
+        hipLaunchKernelGGL((hash_mfma2_kernel<T, Dh>), dim3((unsigned)(nb + ceil_div(also->rows, 64))),
+                           dim3(256), lds, st, hp, *also, (int)nb);
+        SSA_CHECK_LAUNCH();
+        return SSA_OK;
+    }
+    SSA_ALLOW_LDS((hash_mfma_kernel<T, Dh>), lds);
+    hipLaunchKernelGGL((hash_mfma_kernel<T, Dh>), dim3((unsigned)nb), dim3(256), lds, st, hp);
     SSA_CHECK_LAUNCH();
     return SSA_OK;
 }
 
 template <typename T>
-int launch_hash_one(const HashP &hp, int d, hipStream_t st) {
+int launch_hash_one(const HashP &hp, int d, hipStream_t st, const HashP *also = nullptr) {
     if (hp.rows == 0) return SSA_OK;
     if (hp.inj) {
         hipLaunchKernelGGL(hash_kernel<T>, dim3((unsigned)ceil_div(hp.rows, 256)), dim3(256), 0,
@@ -3820,15 +3840,15 @@ int launch_hash_one(const HashP &hp, int d, hipStream_t st) {
         return SSA_OK;
     }
     switch (ssa_pow2_instance(d)) {
-        case 4: return launch_hash_mfma<T, 4>(hp, st);
-        case 8: return launch_hash_mfma<T, 8>(hp, st);
-        case 16: return launch_hash_mfma<T, 16>(hp, st);
-        case 32: return launch_hash_mfma<T, 32>(hp, st);
-        case 64: return launch_hash_mfma<T, 64>(hp, st);
-        case 128: return launch_hash_mfma<T, 128>(hp, st);
-        case 256: return launch_hash_mfma<T, 256>(hp, st);
-        case 512: return launch_hash_mfma<T, 512>(hp, st);
-        case 1024: return launch_hash_mfma<T, 1024>(hp, st);
+        case 4: return launch_hash_mfma<T, 4>(hp, also, st);
+        case 8: return launch_hash_mfma<T, 8>(hp, also, st);
+        case 16: return launch_hash_mfma<T, 16>(hp, also, st);
+        case 32: return launch_hash_mfma<T, 32>(hp, also, st);
+        case 64: return launch_hash_mfma<T, 64>(hp, also, st);
+        case 128: return launch_hash_mfma<T, 128>(hp, also, st);
+        case 256: return launch_hash_mfma<T, 256>(hp, also, st);
+        case 512: return launch_hash_mfma<T, 512>(hp, also, st);
+        case 1024: return launch_hash_mfma<T, 1024>(hp, also, st);
     }
     ssa_set_error("hash: head dim %d", d);
     return SSA_E_UNSUP;
@@ -3846,8 +3866,7 @@ bool key_norm_in_hash(const Dims &D, const ssa_graph_args *a) {
 }
 
 template <typename T>
-int launch_hash(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws,
-                hipStream_t st, bool keys) {
+HashP hash_params(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws, bool keys) {
     HashP hp{};
     hp.planes = a->rand_proj;
     hp.R = D.R; hp.maxP = D.maxP; hp.P = D.P; hp.Tp = D.Tp; hp.NS = D.NS; hp.d = D.d;
@@ -3868,7 +3887,7 @@ int launch_hash(const Dims &D, const ssa_graph_args *a, const Layout &L, char *w
             hp.zero = (uint32_t *)(ws + L.knorm);
             hp.nzero = (int)D.BK;
         }
-        return launch_hash_one<T>(hp, D.d, st);
+        return hp;
     }
     hp.x = a->q.ptr; hp.sb = a->q.sb; hp.sh = a->q.sh; hp.sn = a->q.sn;
     hp.nh = D.Hq; hp.L = D.N; hp.inj = a->q_proj; hp.key_layout = 0;
@@ -3877,14 +3896,18 @@ int launch_hash(const Dims &D, const ssa_graph_args *a, const Layout &L, char *w
     hp.rows = D.BH * D.N;
     // the tie-row counter of the select kernels (replayed once, after every chunk)
     hp.zero1 = (int32_t *)(ws + L.tie_count);
-    return launch_hash_one<T>(hp, D.d, st);
+    return hp;
 }
+
+// Without injected projections, and where no later pass over q hashes it, the
+// query hash rides in the key hash's launch
+template <typename T>
+bool hash_queries_with_keys(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws);
 
 template <typename T, int Dh>
 int launch_rescore(const RsP &rp, int64_t grid, hipStream_t st) {
     const size_t lds = (size_t)(TQ + TC) * ((Dh < 256 ? Dh : 256) + 1) * 4 + (TQ + TC) * 4;
-    SSA_CHECK_HIP(hipFuncSetAttribute((const void *)rescore_kernel<T, Dh>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    SSA_ALLOW_LDS((rescore_kernel<T, Dh>), lds);
     hipLaunchKernelGGL((rescore_kernel<T, Dh>), dim3((unsigned)grid), dim3(256), lds, st, rp);
     SSA_CHECK_LAUNCH();
     return SSA_OK;
@@ -3894,8 +3917,7 @@ template <typename T, int Dh>
 int launch_rescore_mfma(const RsP &rp, int64_t grid, hipStream_t st) {
     // the member ids, rounded up to a whole slice (the slice buffers are static)
     const size_t lds = (size_t)ceil_div(rp.C, RS_SLICE) * RS_SLICE * 4;
-    SSA_CHECK_HIP(hipFuncSetAttribute((const void *)rescore_mfma_kernel<T, Dh>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    SSA_ALLOW_LDS((rescore_mfma_kernel<T, Dh>), lds);
     hipLaunchKernelGGL((rescore_mfma_kernel<T, Dh>), dim3((unsigned)grid), dim3(256), lds, st, rp);
     SSA_CHECK_LAUNCH();
     return SSA_OK;
@@ -3946,8 +3968,7 @@ int rescore_dispatch(int d, const RsP &rp, int64_t grid, hipStream_t st) {
 
 template <typename T, bool LSH, bool CAUSAL, int CAP, bool WIDE>
 int launch_select_w(const SelP &sp, size_t lds, hipStream_t st) {
-    SSA_CHECK_HIP(hipFuncSetAttribute((const void *)select_kernel<T, LSH, CAUSAL, CAP, WIDE>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    SSA_ALLOW_LDS((select_kernel<T, LSH, CAUSAL, CAP, WIDE>), lds);
     const int64_t grid = 8 * ceil_div(sp.nblocks, 8);
     hipLaunchKernelGGL((select_kernel<T, LSH, CAUSAL, CAP, WIDE>), dim3((unsigned)grid),
                        dim3(sp.waves * SSA_WAVE), lds, st, sp);
@@ -4031,8 +4052,7 @@ int launch_replay_pw(const SelP &sp, const Dims &D, int W, uint32_t *rpscr, int 
         return SSA_OK;
     }
     const size_t lds = (size_t)RP_WAVES * rp_lds_words(W, sp.words) * 4;
-    SSA_CHECK_HIP(hipFuncSetAttribute((const void *)topk_replay_kernel<T, LSH, false, CT>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    SSA_ALLOW_LDS((topk_replay_kernel<T, LSH, false, CT>), lds);
     // enough blocks for every resident wave to take a row (the rest exit at once)
     const int64_t blocks = std::min<int64_t>(ceil_div(sp.rows, RP_WAVES), 8192);
     hipLaunchKernelGGL((topk_replay_kernel<T, LSH, false, CT>), dim3((unsigned)blocks),
@@ -4054,13 +4074,22 @@ int launch_replay(const SelP &sp, const Dims &D, uint32_t *rpscr, uint32_t *rpws
         int dev = 0, cus = 0;
         SSA_CHECK_HIP(hipGetDevice(&dev));
         SSA_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        SSA_CHECK_HIP(hipFuncSetAttribute((const void *)topk_replay_wg_kernel<T, LSH>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        SSA_ALLOW_LDS((topk_replay_wg_kernel<T, LSH>), lds);
         // the blocks resident at once (registers and LDS): each loops over its
         // rows; up to four rows per block beat the per-wave replay
+        // (a property of the kernel, the device and its LDS: the last answer is
+        // kept packed in one word, {device + 1, LDS bytes, blocks})
+        static std::atomic<uint64_t> last{0};
         int per_cu = 0;
-        SSA_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, (const void *)topk_replay_wg_kernel<T, LSH>, RPW_THREADS, lds));
+        const uint64_t key = ((uint64_t)(dev + 1) << 40) | ((uint64_t)(uint32_t)lds << 8);
+        const uint64_t kept = last.load(std::memory_order_relaxed);
+        if ((kept & ~(uint64_t)255) == key) {
+            per_cu = (int)(kept & 255);
+        } else {
+            SSA_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, (const void *)topk_replay_wg_kernel<T, LSH>, RPW_THREADS, lds));
+            last.store(key | (uint64_t)std::min(per_cu, 255), std::memory_order_relaxed);
+        }
         const int64_t blocks = std::min<int64_t>(
             std::min<int64_t>(D.rpw_blocks, (int64_t)cus * std::max(1, per_cu)), sp.rows);
         cap = (int)std::min<int64_t>(4 * blocks, sp.rows);
@@ -4068,6 +4097,7 @@ int launch_replay(const SelP &sp, const Dims &D, uint32_t *rpscr, uint32_t *rpws
                            dim3(RPW_THREADS), (size_t)lds, st, sp, chunk, W, D.rpw_nsim, rpwscr,
                            rpw_scratch_words(sp.Call, sp.M, sp.kk, nch), cap);
         SSA_CHECK_LAUNCH();
+        if (sp.rows <= cap) return SSA_OK;     // never more tied rows than it takes
     }
     return rp_wide_ids(sp.words) ? launch_replay_pw<T, LSH, uint32_t>(sp, D, W, rpscr, cap, st)
                                   : launch_replay_pw<T, LSH, uint16_t>(sp, D, W, rpscr, cap, st);
@@ -4122,6 +4152,12 @@ bool aux_hashes_queries(const Dims &D, const ssa_graph_args *a, bool mfma) {
     const int np16 = (int)ceil_div((int64_t)D.R * D.P, 16) * 16;
     return mfma && !a->q_proj && (uintptr_t)a->rand_proj % 16 == 0 &&
            (size_t)4 * 16 * (np16 + 1) * 4 <= 48 * 1024;
+}
+
+template <typename T>
+bool hash_queries_with_keys(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws) {
+    return !D.fused && !a->k_proj && !a->q_proj && D.BK * D.M > 0 && D.BH * D.N > 0 &&
+           !aux_hashes_queries<T>(D, a, rescore_uses_mfma<T>(D.d, rescore_common(D, a, L, ws)));
 }
 
 // The first head chunk's aux pass runs beside the key sort's top levels
@@ -4215,7 +4251,7 @@ int launch_sort_aux(const Dims &D, const ssa_graph_args *a, const Layout &L, cha
         case 128: fn = (const void *)sort_aux_kernel<T, 128>; break;
         default: ssa_set_error("sort and aux: head dim %d", D.d); return SSA_E_UNSUP;
     }
-    SSA_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    SSA_ALLOW_LDS((fn), lds);
     switch (mfma_instance(D.d)) {
 #define SSA_SORT_AUX(DD)                                                                     \
     case DD:                                                                                 \
@@ -4236,8 +4272,7 @@ int launch_sort_aux(const Dims &D, const ssa_graph_args *a, const Layout &L, cha
     const int64_t nhist = D.dense ? 0 : (int64_t)qp.ninst * nqb;
     const size_t hl = std::max<size_t>((size_t)SEG_WAVES * seg_lds_words<uint16_t>() * 4,
                                        (size_t)D.NB * 4);
-    SSA_CHECK_HIP(hipFuncSetAttribute((const void *)sort_seg_hist_kernel,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)hl));
+    SSA_ALLOW_LDS((sort_seg_hist_kernel), hl);
     hipLaunchKernelGGL(sort_seg_hist_kernel, dim3((unsigned)(nseg + nhist)),
                        dim3(256), hl, st, sa, qp, nseg, nqb);
     SSA_CHECK_LAUNCH();
@@ -4250,7 +4285,15 @@ int keys_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws
     int rc = SSA_OK;
     {
         // (fused: the key projection wrote the key ids and the 16-row norm maxima)
-        if (!D.fused) rc = launch_hash<T>(D, a, L, ws, st, true);
+        if (!D.fused) {
+            const HashP kp = hash_params<T>(D, a, L, ws, true);
+            if (hash_queries_with_keys<T>(D, a, L, ws)) {
+                const HashP qp = hash_params<T>(D, a, L, ws, false);
+                rc = launch_hash_one<T>(kp, D.d, st, &qp);
+            } else {
+                rc = launch_hash_one<T>(kp, D.d, st);
+            }
+        }
         if (rc) return rc;
         // max |k|^2 per (batch, kv head): the query code scales derive from it
         KnP kp{};
@@ -4341,16 +4384,13 @@ int keys_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws
             // beside the first chunk's bucket scan (its histogram ran beside
             // the segments)
             const QbP qp = qb_params(D, a, L, ws, 0, (int)std::min<int64_t>(D.BH, D.nbh_chunk));
-            SSA_CHECK_HIP(hipFuncSetAttribute((const void *)list_sort_scan_kernel,
-                                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                                              (int)lds));
+            SSA_ALLOW_LDS((list_sort_scan_kernel), lds);
             hipLaunchKernelGGL(list_sort_scan_kernel, dim3((unsigned)(nls + qp.ninst)), dim3(256),
                                lds, st, lp, qp, (int)nls);
             SSA_CHECK_LAUNCH();
             return SSA_OK;
         }
-        SSA_CHECK_HIP(hipFuncSetAttribute((const void *)list_sort_kernel,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        SSA_ALLOW_LDS((list_sort_kernel), lds);
         hipLaunchKernelGGL(list_sort_kernel, dim3((unsigned)nls), dim3(256), lds, st, lp);
         SSA_CHECK_LAUNCH();
         if (sort_aux) {
@@ -4463,8 +4503,8 @@ int queries_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char 
     const bool mfma = rescore_uses_mfma<T>(D.d, rp);
     const bool fuse_qhash = aux_hashes_queries<T>(D, a, mfma);
     int rc = SSA_OK;
-    if (!fuse_qhash && !D.fused) {
-        rc = launch_hash<T>(D, a, L, ws, st, false);
+    if (!fuse_qhash && !D.fused && !hash_queries_with_keys<T>(D, a, L, ws)) {
+        rc = launch_hash_one<T>(hash_params<T>(D, a, L, ws, false), D.d, st);
         if (rc) return rc;
     }
     SelP last{};

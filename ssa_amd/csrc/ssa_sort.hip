@@ -162,8 +162,7 @@ static int launch_sort(const uint16_t *ids, int rows, int n, int NB, int32_t *pe
     int4 *segs = (int4 *)(t + al256(rn * (int64_t)sizeof(W)));
     int *segcount = ssa_sort_counter((uint16_t *)t, rows, n);
     unsigned char *glb = (unsigned char *)t + al256(rn * (int64_t)sizeof(W)) + al256(rn * 16) + 256;
-    SSA_CHECK_HIP(hipFuncSetAttribute((const void *)sort_top_kernel<Pos>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    SSA_ALLOW_LDS((sort_top_kernel<Pos>), lds);
     hipLaunchKernelGGL((sort_top_kernel<Pos>), dim3(rows), dim3(SORT_THREADS), lds, st, ids, n, NB,
                        perm, bstart, bsize, gkv, segs, segcount, glb, tl, cap);
     SSA_CHECK_LAUNCH();

@@ -223,7 +223,7 @@ class _GatherAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, neighbors, valid, scale, fp32w, dropout_p, seed, row_invalid=None):
         out = _lib.gather_attention_fwd(q, k, v, neighbors, valid, scale, fp32w, dropout_p, seed,
-                                        row_invalid=row_invalid)
+                                        row_invalid=row_invalid, _checked=True)
         ctx.save_for_backward(q, k, v, neighbors, valid)
         ctx.cfg = (scale, fp32w, dropout_p, seed)
         return out
