@@ -31,8 +31,10 @@ apply_fwd_kernel(ApplyP p) {
     if (row >= p.rows) return;
     const int lane = lane_id();
     const int sub = lane / LPR, li = lane % LPR;
-    int32_t *ix = reinterpret_cast<int32_t *>(smem) + (int64_t)wid * 2 * p.K;   // key ids, -1 = masked
-    float *sc = reinterpret_cast<float *>(ix + p.K);                          // scores, then p
+    constexpr int STEP = RPI * U;
+    const int Kp = (p.K + STEP - 1) / STEP * STEP;                            // padded slots
+    int32_t *ix = reinterpret_cast<int32_t *>(smem) + (int64_t)wid * 2 * Kp;    // key ids, -1 = masked
+    float *sc = reinterpret_cast<float *>(ix + Kp);                           // scores, then p
 
     const int n = (int)(row % p.N);
     const int64_t bh = row / p.N;
@@ -59,7 +61,7 @@ apply_fwd_kernel(ApplyP p) {
     // graph); an out-of-range id marked valid is skipped here but not counted
     int ninv = 0;
     auto slots = [&](auto i32) __attribute__((always_inline)) {
-        for (int j0 = 0; j0 < p.K; j0 += APPLY_SLOT_BATCH * SSA_WAVE) {
+        for (int j0 = 0; j0 < Kp; j0 += APPLY_SLOT_BATCH * SSA_WAVE) {
             RowSlots<APPLY_SLOT_BATCH, decltype(i32)::value> rs;
             rs.load(p, row, nb, va, j0, lane);
 #pragma unroll
@@ -68,7 +70,7 @@ apply_fwd_kernel(ApplyP p) {
                 const bool in = j < p.K;
                 const bool marked = in && rs.marked(u);
                 const int64_t x = rs.y[u];
-                if (in) ix[j] = (!marked && x >= 0 && x < p.M) ? (int)x : -1;
+                if (j < Kp) ix[j] = (in && !marked && x >= 0 && x < p.M) ? (int)x : -1;
                 ninv += __popcll(wave_ballot(marked));
             }
         }
@@ -82,28 +84,25 @@ apply_fwd_kernel(ApplyP p) {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
-    // ---- scores
-    for (int j0 = 0; j0 < p.K; j0 += RPI * U) {
+    // ---- scores (masked slots are set to -inf by the softmax); the lanes' sums
+    // by DPP, whose tree is the shuffles' (no LDS round trips per row: 131 -> 96 us
+    // at 73,488 fp32 rows of 54 slots, d = 64)
+    for (int j0 = 0; j0 < Kp; j0 += STEP) {
         int xi[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int j = j0 + u * RPI + sub;
-            xi[u] = j < p.K ? ix[j] : -1;
-        }
+        for (int u = 0; u < U; ++u) xi[u] = ix[j0 + u * RPI + sub];
         float kf[U][VEC];
 #pragma unroll
         for (int u = 0; u < U; ++u)
             load_vec<T, VEC>(kb + (int64_t)(xi[u] < 0 ? 0 : xi[u]) * p.ksn + lofs, kf[u]);
+        float part[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            float part = 0.f;
+            part[u] = 0.f;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) part = fmaf(qf[e], kf[u][e], part);
-#pragma unroll
-            for (int o = LPR / 2; o > 0; o >>= 1) part += __shfl_xor(part, o, SSA_WAVE);
-            const int j = j0 + u * RPI + sub;
-            if (li == 0 && j < p.K) sc[j] = xi[u] >= 0 ? part * p.scale : -INFINITY;
+            for (int e = 0; e < VEC; ++e) part[u] = fmaf(qf[e], kf[u][e], part[u]);
         }
+        rows_to_lds<LPR, RPI, U>(part, li, sub, sc + j0, p.scale);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -112,18 +111,25 @@ apply_fwd_kernel(ApplyP p) {
     // ---- fp32 softmax, p computed once per slot (rounded to the value dtype
     // unless fp32_attn_weights; inverted dropout applied to p)
     float m = -INFINITY;
-    for (int j = lane; j < p.K; j += SSA_WAVE) m = fmaxf(m, sc[j]);
+    for (int j = lane; j < p.K; j += SSA_WAVE) {
+        const float s = ix[j] >= 0 ? sc[j] : -INFINITY;
+        sc[j] = s;
+        m = fmaxf(m, s);
+    }
     m = wave_max(m);
     float l = 0.f;
     for (int j = lane; j < p.K; j += SSA_WAVE) l += expf(sc[j] - m);
     l = wave_sum(l);
     const float inv = 1.f / l;
-    for (int j = lane; j < p.K; j += SSA_WAVE) {
-        float w = expf(sc[j] - m) * inv;
-        if (!p.fp32w) w = Cvt<T>::round(w);
-        if (p.drop_p > 0.f) {
-            w = (drop_uniform(p.seed, row, j) < p.drop_p) ? 0.f : w * drop_scale_of<T>(p);
+    for (int j = lane; j < Kp; j += SSA_WAVE) {
+        float w = 0.f;
+        if (j < p.K) {
+            w = expf(sc[j] - m) * inv;
             if (!p.fp32w) w = Cvt<T>::round(w);
+            if (p.drop_p > 0.f) {
+                w = (drop_uniform(p.seed, row, j) < p.drop_p) ? 0.f : w * drop_scale_of<T>(p);
+                if (!p.fp32w) w = Cvt<T>::round(w);
+            }
         }
         sc[j] = w;
     }
@@ -135,15 +141,13 @@ apply_fwd_kernel(ApplyP p) {
     float acc[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
-    for (int j0 = 0; j0 < p.K; j0 += RPI * U) {
+    for (int j0 = 0; j0 < Kp; j0 += STEP) {
         int xi[U];
         float pj[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int j = j0 + u * RPI + sub;
-            const bool in = j < p.K;
-            xi[u] = in ? ix[j] : -1;
-            pj[u] = in ? sc[j] : 0.f;
+            xi[u] = ix[j0 + u * RPI + sub];
+            pj[u] = sc[j0 + u * RPI + sub];
         }
         float vf[U][VEC];
 #pragma unroll
@@ -693,7 +697,6 @@ int launch_apply(const ApplyP &p, hipStream_t st, bool bwd) {
         hipLaunchKernelGGL((apply_bwd_kernel<T, D>), dim3((unsigned)grid),
                            dim3(WAVES * SSA_WAVE), lds, st, p);
     } else {
-        const size_t lds = (size_t)WAVES * 2 * p.K * sizeof(float);
         // slot batches of 8 row loads, 4 where a load covers 16 rows or more
         // (64 slots a step at 8 rows a load: 64-wide bf16 heads 1% faster)
         constexpr int U = (Geo<T, D>::RPI >= 16) ? 4 : 8;
@@ -711,11 +714,13 @@ int launch_apply(const ApplyP &p, hipStream_t st, bool bwd) {
                 return SSA_OK;
             }
         }
-        if (lds > 65536)
+        constexpr int UF = Geo<T, D>::RPI * U;
+        const size_t ldsf = (size_t)WAVES * 2 * ceil_div(p.K, UF) * UF * sizeof(float);
+        if (ldsf > 65536)
             SSA_CHECK_HIP(hipFuncSetAttribute((const void *)apply_fwd_kernel<T, D, U>,
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsf));
         hipLaunchKernelGGL((apply_fwd_kernel<T, D, U>), dim3((unsigned)grid),
-                           dim3(WAVES * SSA_WAVE), lds, st, p);
+                           dim3(WAVES * SSA_WAVE), ldsf, st, p);
     }
     SSA_CHECK_LAUNCH();
     return SSA_OK;

@@ -271,6 +271,70 @@ __device__ __forceinline__ float butterfly_rows(float (&v)[U], int li) {
     return y + dpp_move<0xB1>(y);                       // quad perm [1,0,3,2]: li ^ 1
 }
 
+// Sum over the L lanes of each aligned group as xor shuffles by L / 2, .., 1
+// add them (that tree's rounding, which long and unvectorised rows have too):
+// once the step by 16 has run, rotating a row of 16 lanes by 8, 4, 2 and 1
+// brings a lane the same partner value as the xor.
+template <int L>
+__device__ __forceinline__ float tree_sum(float v) {
+    if constexpr (L > 32) return wave_sum(v);
+    if constexpr (L >= 32) v += __shfl_xor(v, 16, SSA_WAVE);
+    if constexpr (L >= 16) v = dpp_add<0x128>(v);        // row_ror:8
+    if constexpr (L >= 16) v = dpp_add<0x124>(v);        // row_ror:4
+    if constexpr (L == 8) v += dpp_move<0x1B>(dpp_move<0x141>(v));   // li ^ 7, then ^ 3
+    if constexpr (L >= 4) v = dpp_add<0x4E>(v);          // li ^ 2
+    if constexpr (L >= 2) v = dpp_add<0xB1>(v);          // li ^ 1
+    return v;
+}
+
+// butterfly_rows with the pairings of tree_sum (li ^ 8, ^ 4, ^ 2, ^ 1), so each
+// row's total is that tree's, bit for bit
+template <int U>
+__device__ __forceinline__ float tree_rows(float (&v)[U], int li) {
+    static_assert(U == 4 || U == 8, "over 8 or 16 lanes");
+    float w[4];
+    if constexpr (U == 8) {
+        const bool hi = li >= 8;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float send = hi ? v[k] : v[k + 4], keep = hi ? v[k + 4] : v[k];
+            w[k] = keep + dpp_move<0x128>(send);         // row_ror:8
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = v[k];
+    }
+    float x[2];
+    {
+        const bool hi = (li & 4) != 0;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float send = hi ? w[k] : w[k + 2], keep = hi ? w[k + 2] : w[k];
+            x[k] = keep + dpp_move<0x1B>(dpp_move<0x141>(send));
+        }
+    }
+    const bool hi = (li & 2) != 0;
+    const float send = hi ? x[0] : x[1], keep = hi ? x[1] : x[0];
+    float y = keep + dpp_move<0x4E>(send);
+    return y + dpp_move<0xB1>(y);
+}
+
+// sums of v[u] over each row's LPR lanes, stored to dst[row slot u * RPI + sub]
+template <int LPR, int RPI, int U>
+__device__ __forceinline__ void rows_to_lds(float (&v)[U], int li, int sub, float *dst, float mul) {
+    if constexpr (2 * U == LPR && (U == 4 || U == 8)) {
+        const float t = tree_rows<U>(v, li);
+        const int r = (U == 8 ? 4 * (li >= 8) : 0) + 2 * ((li & 4) != 0) + ((li & 2) != 0);
+        if ((li & 1) == 0) dst[r * RPI + sub] = t * mul;
+    } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float t = tree_sum<LPR>(v[u]);
+            if (li == 0) dst[u * RPI + sub] = t * mul;
+        }
+    }
+}
+
 // checks the forward's arguments and fills p
 inline int check_view(const ssa_tensor4 &t, int dtype, const char *name) {
     if (!t.ptr) { ssa_set_error("%s: null pointer", name); return SSA_E_ARG; }
