@@ -4263,18 +4263,86 @@ int launch_sort_aux(const Dims &D, const ssa_graph_args *a, const Layout &L, cha
 #undef SSA_SORT_AUX
     }
     SSA_CHECK_LAUNCH();
+    if (D.dense) return SSA_OK;        // the segments run beside the scores
     // the segments, beside the first chunk's query histogram (its ids came
     // from the launch above)
     static_assert(SEG_WAVES * SSA_WAVE == 256, "the query histogram takes 256 queries a block");
     const QbP qp = qb_params(D, a, L, ws, 0, nbh);
     const int nseg = ssa_sort_seg_blocks(sa.rows, sa.n);
     const int nqb = (int)ceil_div(D.N, 256);
-    const int64_t nhist = D.dense ? 0 : (int64_t)qp.ninst * nqb;
     const size_t hl = std::max<size_t>((size_t)SEG_WAVES * seg_lds_words<uint16_t>() * 4,
                                        (size_t)D.NB * 4);
     SSA_ALLOW_LDS((sort_seg_hist_kernel), hl);
-    hipLaunchKernelGGL(sort_seg_hist_kernel, dim3((unsigned)(nseg + nhist)),
+    hipLaunchKernelGGL(sort_seg_hist_kernel, dim3((unsigned)(nseg + (int64_t)qp.ninst * nqb)),
                        dim3(256), hl, st, sa, qp, nseg, nqb);
+    SSA_CHECK_LAUNCH();
+    return SSA_OK;
+}
+
+// dense form: the codes of every (query, key) score of the head chunk
+// [bh0, bh0 + nbh), beside the key sort's segments when given
+template <typename T>
+int launch_dense(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws, int64_t bh0,
+                 int nbh, bool mfma, const SortTopArgs *segs, hipStream_t st) {
+    DnP dp{};
+    dp.q = a->q.ptr; dp.k = a->k.ptr;
+    dp.qsb = a->q.sb; dp.qsh = a->q.sh; dp.qsn = a->q.sn;
+    dp.ksb = a->k.sb; dp.ksh = a->k.sh; dp.ksn = a->k.sn;
+    dp.S = (uint32_t *)(ws + L.S);
+    const AuxP ap = aux_params(D, a, L, ws, bh0, nbh, false);
+    dp.aux = ap.out; dp.NA = ap.NA;
+    dp.knorm = (const uint32_t *)(ws + L.knorm);
+    if (key_norm_in_hash(D, a)) {
+        dp.kpart = (const uint32_t *)(ws + L.kpart);
+        dp.kp_n = D.M / 16;
+    }
+    dp.N = D.N; dp.M = D.M; dp.Ms = D.Ms; dp.Hq = D.Hq; dp.Hkv = D.Hkv; dp.rep = D.rep;
+    dp.bh0 = (int)bh0; dp.nbh = nbh; dp.causal = a->causal ? 1 : 0; dp.d = D.d;
+    dp.ktiles = (int)ceil_div(D.M, mfma ? DM_K : DV_T);
+    const bool wide = ceil_div(D.N, 64 * DM_QF) * dp.ktiles * nbh >= DM_TILES;
+    dp.qtiles = (int)ceil_div(D.N, !mfma ? DV_T : 64 * (wide ? DM_QF : DM_QF / 2));
+    static_assert(SEG_WAVES * SSA_WAVE == 256, "segments and tiles share a launch");
+    SortTopArgs sa{};
+    int nseg = 0;
+    size_t lds = mfma ? 0 : DV_LDS;
+    const int64_t tiles = (int64_t)dp.qtiles * dp.ktiles * nbh;
+    // A shared launch pays where the tiles outlast the segments or all fit the
+    // chip at once; few long tiles would wait for the slots of the segments'
+    // workgroups, which take the tiles' registers (512 tiles behind 384
+    // segment workgroups: 107 us against 24 + 45 apart).
+    const bool share = segs && (tiles >= 1024 || tiles + ssa_sort_seg_blocks(segs->rows, segs->n) <= 256);
+    if (segs && !share) {
+        const int rc = ssa_launch_sort_seg(*segs, st);
+        if (rc) return rc;
+    }
+    if (share) {
+        sa = *segs;
+        nseg = (int)ceil_div(ssa_sort_seg_blocks(sa.rows, sa.n), 8) * 8;
+        lds = std::max<size_t>(lds, (size_t)SEG_WAVES * seg_lds_words<uint16_t>() * 4);
+    }
+    const unsigned grid = (unsigned)(nseg + 8 * ceil_div(tiles, 8));
+    if constexpr (!std::is_same<T, float>::value) {
+        if (mfma) {
+#define SSA_DENSE(DD)                                                                              \
+    case DD:                                                                                       \
+        if (wide)                                                                                  \
+            hipLaunchKernelGGL((dense_mfma_kernel<T, DD, DM_QF>), dim3(grid), dim3(256), lds, st,  \
+                               dp, sa, nseg);                                                      \
+        else                                                                                       \
+            hipLaunchKernelGGL((dense_mfma_kernel<T, DD, DM_QF / 2>), dim3(grid), dim3(256), lds,  \
+                               st, dp, sa, nseg);                                                  \
+        break;
+            switch (mfma_instance(D.d)) {
+                SSA_DENSE(8) SSA_DENSE(16) SSA_DENSE(32) SSA_DENSE(64) SSA_DENSE(96) SSA_DENSE(128)
+                default: ssa_set_error("dense scores: head dim %d", D.d); return SSA_E_UNSUP;
+            }
+#undef SSA_DENSE
+            SSA_CHECK_LAUNCH();
+            return SSA_OK;
+        }
+    }
+    SSA_ALLOW_LDS((dense_valu_kernel<T>), lds);
+    hipLaunchKernelGGL((dense_valu_kernel<T>), dim3(grid), dim3(256), lds, st, dp, sa, nseg);
     SSA_CHECK_LAUNCH();
     return SSA_OK;
 }
@@ -4325,6 +4393,37 @@ int keys_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws
     }
     // the key hash cleared the sort's counter
     bool done = false;
+    SortTopArgs sa{};
+    if (D.dense && !D.fused) {
+        // (fused: the queries are not projected yet.)  The sort's top levels; then the segments beside the first head chunk's
+        // scores, which need the aux pass's code scales on the matrix cores
+        const int nbh = (int)std::min<int64_t>(D.BH, D.nbh_chunk);
+        const bool mfma = rescore_uses_mfma<T>(D.d, rescore_common(D, a, L, ws));
+        rc = ssa_sort_top_setup((const uint16_t *)(ws + L.kid), (int)(D.BK * D.R), D.M, D.P,
+                                (int32_t *)(ws + L.perm), (int32_t *)(ws + L.bstart),
+                                (int32_t *)(ws + L.bsize), (uint16_t *)(ws + L.sorttmp), &sa);
+        if (rc) return rc;
+        if constexpr (!std::is_same<T, float>::value) {
+            if (sort_aux) {
+                rc = launch_sort_aux<T>(D, a, L, ws, st);
+                done = true;
+            }
+        }
+        if (!done) rc = ssa_launch_sort_top(sa, st);
+        if (rc) return rc;
+        if (!done && mfma) {
+            AuxP ap = aux_params(D, a, L, ws, 0, nbh, aux_hashes_queries<T>(D, a, mfma));
+            if (key_norm_in_hash(D, a)) {
+                ap.kpart = (const uint32_t *)(ws + L.kpart);
+                ap.kp_n = D.M / 16;
+            }
+            rc = aux_dispatch<T>(D.d, mfma, ap, st);
+            if (rc) return rc;
+        }
+        rc = launch_dense<T>(D, a, L, ws, 0, nbh, mfma, &sa, st);
+        if (rc) return rc;
+        done = true;
+    } else
     if constexpr (!std::is_same<T, float>::value) {
         if (sort_aux) {
             rc = launch_sort_aux<T>(D, a, L, ws, st);
@@ -4434,47 +4533,6 @@ SelP select_common(const Dims &D, const ssa_graph_args *a, const Layout &L, char
     return sp;
 }
 
-// dense form: the codes of every (query, key) score of a head chunk
-template <typename T>
-int dense_scores(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws, SelP &sp,
-                 hipStream_t st) {
-    sp.S32 = (const uint32_t *)(ws + L.S);
-    sp.lbits = (const uint64_t *)(ws + L.lbits);
-    sp.lmax = (const int32_t *)(ws + L.lmax);
-    sp.knorm = (const uint32_t *)(ws + L.knorm);
-    sp.Ms = D.Ms; sp.nw = D.nw;
-    auto magic = [](int d) { return (uint32_t)((((uint64_t)1 << 32) + d - 1) / d); };
-    sp.magN = magic(D.N); sp.magHq = magic(D.Hq); sp.magRep = magic(D.rep); sp.magNS = magic(D.NS);
-    DnP dp{};
-    dp.q = a->q.ptr; dp.k = a->k.ptr;
-    dp.qsb = a->q.sb; dp.qsh = a->q.sh; dp.qsn = a->q.sn;
-    dp.ksb = a->k.sb; dp.ksh = a->k.sh; dp.ksn = a->k.sn;
-    dp.S = (uint32_t *)(ws + L.S);
-    dp.aux = sp.aux; dp.knorm = sp.knorm; dp.NA = sp.NA;
-    dp.N = D.N; dp.M = D.M; dp.Ms = D.Ms; dp.Hq = D.Hq; dp.Hkv = D.Hkv; dp.rep = D.rep;
-    dp.bh0 = sp.bh0; dp.nbh = (int)(sp.rows / D.N); dp.causal = a->causal ? 1 : 0; dp.d = D.d;
-    const bool mfma = sp.mfma != 0;
-    dp.qtiles = (int)ceil_div(D.N, mfma ? DM_Q : DV_T);
-    dp.ktiles = (int)ceil_div(D.M, mfma ? DM_K : DV_T);
-    const unsigned grid = (unsigned)(8 * ceil_div((int64_t)dp.qtiles * dp.ktiles * dp.nbh, 8));
-    if constexpr (!std::is_same<T, float>::value) {
-        if (mfma) {
-#define SSA_DENSE(DD) \
-    case DD: hipLaunchKernelGGL((dense_mfma_kernel<T, DD>), dim3(grid), dim3(256), 0, st, dp); break;
-            switch (mfma_instance(D.d)) {
-                SSA_DENSE(8) SSA_DENSE(16) SSA_DENSE(32) SSA_DENSE(64) SSA_DENSE(96) SSA_DENSE(128)
-                default: ssa_set_error("dense scores: head dim %d", D.d); return SSA_E_UNSUP;
-            }
-#undef SSA_DENSE
-            SSA_CHECK_LAUNCH();
-            return SSA_OK;
-        }
-    }
-    hipLaunchKernelGGL((dense_valu_kernel<T>), dim3(grid), dim3(256), 0, st, dp);
-    SSA_CHECK_LAUNCH();
-    return SSA_OK;
-}
-
 template <typename T, bool CAUSAL>
 int dense_select_c(const SelP &sp0, hipStream_t st) {
     SelP sp = sp0;
@@ -4515,15 +4573,24 @@ int queries_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char 
         // writes, and the query buckets need the ids it writes when fused
         // (the first chunk's ran beside the key sort when sort_aux)
         const AuxP ap = aux_params(D, a, L, ws, bh0, nbh, fuse_qhash);
-        // (dense without the matrix cores: the score kernel takes the scales)
-        if (!D.fused && !(sort_aux && bh0 == 0) && (mfma || !D.dense))
+        // (dense: the first chunk's ran in the key phase, and without the matrix
+        // cores the score kernel takes the scales)
+        if (!D.fused && !((sort_aux || D.dense) && bh0 == 0) && (mfma || !D.dense))
             rc = aux_dispatch<T>(D.d, mfma, ap, st);
         if (rc) return rc;
         if (D.dense) {
             SelP sp = select_common<T>(D, a, L, ws, bh0, nbh, mfma);
             sp.aux = mfma ? ap.out : nullptr;
             sp.NA = ap.NA;
-            rc = dense_scores<T>(D, a, L, ws, sp, st);
+            sp.S32 = (const uint32_t *)(ws + L.S);
+            sp.lbits = (const uint64_t *)(ws + L.lbits);
+            sp.lmax = (const int32_t *)(ws + L.lmax);
+            sp.knorm = (const uint32_t *)(ws + L.knorm);
+            sp.Ms = D.Ms; sp.nw = D.nw;
+            auto magic = [](int d) { return (uint32_t)((((uint64_t)1 << 32) + d - 1) / d); };
+            sp.magN = magic(D.N); sp.magHq = magic(D.Hq); sp.magRep = magic(D.rep); sp.magNS = magic(D.NS);
+            // (the first chunk's scores ran beside the key sort unless fused)
+            if (bh0 > 0 || D.fused) rc = launch_dense<T>(D, a, L, ws, bh0, nbh, mfma, nullptr, st);
             if (!rc) rc = dense_select<T>(sp, st);
             if (rc) return rc;
             last = sp;

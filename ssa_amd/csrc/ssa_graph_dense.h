@@ -34,7 +34,10 @@ struct DnP {
     int64_t qsb, qsh, qsn, ksb, ksh, ksn;
     uint32_t *S;           // (nbh * N, Ms / 2)
     const float *aux;      // MFMA: the query's code scale, last of NA floats
-    const uint32_t *knorm; // VALU: max |k|^2 per (batch, kv head), float bits
+    // VALU: max |k|^2 per (batch, kv head), float bits, or the key hash's 16-row
+    // maxima (kp_n per kv head)
+    const uint32_t *knorm, *kpart;
+    int kp_n;
     int NA;
     int N, M, Ms, Hq, Hkv, rep, bh0, nbh, causal, d;
     int qtiles, ktiles;    // workgroup tiles over queries and keys
@@ -95,12 +98,14 @@ __global__ void __launch_bounds__(1024) list_bits_kernel(LbP p) {
 }
 
 // ---------------------------------------------------------------- scores
-constexpr int DM_QF = 4;               // 16-query operands per wave
-constexpr int DM_Q = 64 * DM_QF;       // queries per workgroup
+// 16-query operands per wave (QF): 4, or 2 where 4 leaves fewer than DM_TILES
+// workgroups (64 x 2,048 queries over 512 keys, d = 64: 512 workgroups 69 us,
+// 1,024 of half the queries 50 us)
+constexpr int DM_QF = 4, DM_TILES = 1024;
 constexpr int DM_K = 512;              // keys per workgroup: 4 blocks
 
 // 16-bit q and k on the matrix cores, with the k steps, operand roles and so
-// the sums of the list form's rescore.  A wave holds 64 queries as B operands
+// the sums of the list form's rescore.  A wave holds 16 QF queries as B operands
 // and walks its keys in pairs of 16-row tiles 64 keys apart, whose results are
 // the four 32-bit pairs a lane stores with one 16-byte store; the next pair's K
 // rows load while this one multiplies.  K rows come straight from the L1 (the
@@ -109,32 +114,32 @@ constexpr int DM_K = 512;              // keys per workgroup: 4 blocks
 // behind the next block's first loads.  Bound: the K fragments' way through the
 // L1 (64 queries a wave instead of 32, which halves them: 95 -> 72 us at 16 heads
 // of 2,999 causal rows, d = 96; 0.14 GB of codes).
-template <typename T, int D>
-__global__ void __launch_bounds__(256) dense_mfma_kernel(DnP p) {
+template <typename T, int D, int QF>
+__device__ __forceinline__ void dense_mfma_tile(const DnP &p, int64_t phys) {
     using V = typename Mfma16<T>::vec;
     constexpr int KS = (D + 31) / 32;
     const int64_t tiles = (int64_t)p.qtiles * p.ktiles;
-    const int64_t blk = xcd_logical_block(blockIdx.x, tiles * p.nbh);
+    const int64_t blk = xcd_logical_block(phys, tiles * p.nbh);
     if (blk >= tiles * p.nbh) return;
     const int bhl = (int)(blk / tiles);
     const int t = (int)(blk % tiles);
     const int qt = t / p.ktiles, kt = t % p.ktiles;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / SSA_WAVE);
-    const int n0 = qt * DM_Q + 16 * DM_QF * wid;
+    const int n0 = qt * 64 * QF + 16 * QF * wid;
     const int k0 = kt * DM_K;
     // causal: keys up to the wave's last query
     int kend = min(k0 + DM_K, (p.M + DN_BLK - 1) / DN_BLK * DN_BLK);
-    if (p.causal) kend = min(kend, (min(n0 + 16 * DM_QF - 1, p.N - 1) / DN_BLK + 1) * DN_BLK);
+    if (p.causal) kend = min(kend, (min(n0 + 16 * QF - 1, p.N - 1) / DN_BLK + 1) * DN_BLK);
     if (n0 >= p.N || k0 >= kend) return;
     const int bh = p.bh0 + bhl, b = bh / p.Hq, h = bh % p.Hq, g = h / p.rep;
     const int lane = lane_id(), li = lane % 16, lg = lane / 16;
     const T *qbase = (const T *)p.q + b * p.qsb + h * p.qsh;
     const T *kbase = (const T *)p.k + b * p.ksb + g * p.ksh;
     const V zero = __builtin_bit_cast(V, make_uint4(0, 0, 0, 0));
-    V qf[DM_QF][KS];
-    float sc[DM_QF];
+    V qf[QF][KS];
+    float sc[QF];
 #pragma unroll
-    for (int i = 0; i < DM_QF; ++i) {
+    for (int i = 0; i < QF; ++i) {
         const int n = min(n0 + 16 * i + li, p.N - 1);
         sc[i] = p.aux[((int64_t)bhl * p.N + n) * p.NA + p.NA - 1];
 #pragma unroll
@@ -157,10 +162,10 @@ __global__ void __launch_bounds__(256) dense_mfma_kernel(DnP p) {
         }
     };
     uint32_t *srow = p.S + ((int64_t)bhl * p.N + n0 + li) * (p.Ms / 2) + 4 * lg;
-    uint4 w[4][DM_QF];                     // the block's codes: tile pair, 16 queries
-    auto score = [&](const V (&a)[2][KS], uint4 (&o)[DM_QF]) __attribute__((always_inline)) {
+    uint4 w[4][QF];                     // the block's codes: tile pair, 16 queries
+    auto score = [&](const V (&a)[2][KS], uint4 (&o)[QF]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < DM_QF; ++i) {
+        for (int i = 0; i < QF; ++i) {
             f32x4_t c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0;
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
@@ -185,7 +190,7 @@ __global__ void __launch_bounds__(256) dense_mfma_kernel(DnP p) {
         load(min(x + DN_BLK, kend - DN_BLK), a0);
         score(a1, w[3]);
 #pragma unroll
-        for (int i = 0; i < DM_QF; ++i)
+        for (int i = 0; i < QF; ++i)
             if (n0 + 16 * i + li < p.N)
 #pragma unroll
                 for (int a = 0; a < 4; ++a)
@@ -201,12 +206,12 @@ constexpr int DV_LD = DV_T + 4;
 // tiles, 8 queries x 8 keys per thread, each score one fmaf chain over the
 // head dim in order, as the exact keys run it.  Bound: fp32 FMA issue (64 FMAs
 // per four 16-byte LDS reads).
+constexpr int DV_LDS = (2 * DV_C * DV_LD + DV_T) * 4;
 template <typename T>
-__global__ void __launch_bounds__(256) dense_valu_kernel(DnP p) {
-    __shared__ __align__(16) float Qs[DV_C * DV_LD], Ks[DV_C * DV_LD];
-    __shared__ float q2s[DV_T];
+__device__ __forceinline__ void dense_valu_tile(const DnP &p, int64_t phys, float *lds) {
+    float *Qs = lds, *Ks = Qs + DV_C * DV_LD, *q2s = Ks + DV_C * DV_LD;
     const int64_t tiles = (int64_t)p.qtiles * p.ktiles;
-    const int64_t blk = xcd_logical_block(blockIdx.x, tiles * p.nbh);
+    const int64_t blk = xcd_logical_block(phys, tiles * p.nbh);
     if (blk >= tiles * p.nbh) return;
     const int bhl = (int)(blk / tiles);
     const int t = (int)(blk % tiles);
@@ -249,7 +254,18 @@ __global__ void __launch_bounds__(256) dense_valu_kernel(DnP p) {
                 for (int j = 0; j < 8; ++j) acc[i][j] = fmaf(qv[i], kv[j], acc[i][j]);
         }
     }
-    if (tid < DV_T) q2s[tid] = code_scale(q2, __uint_as_float(p.knorm[b * p.Hkv + g]));
+    if (tid < DV_T) {
+        uint32_t kn;
+        if (p.kpart) {
+            const uint32_t *kt = p.kpart + (int64_t)(b * p.Hkv + g) * p.kp_n;
+            uint32_t m = 0u;
+            for (int i = lane_id(); i < p.kp_n; i += SSA_WAVE) m = max(m, kt[i]);
+            kn = wave_max_u(m);
+        } else {
+            kn = p.knorm[b * p.Hkv + g];
+        }
+        q2s[tid] = code_scale(q2, __uint_as_float(kn));
+    }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -263,6 +279,30 @@ __global__ void __launch_bounds__(256) dense_valu_kernel(DnP p) {
         w.w = dn_pair(acc[i][3], acc[i][7], sc);
         *reinterpret_cast<uint4 *>(p.S + ((int64_t)bhl * p.N + n) * (p.Ms / 2) + k0 / 2 + 4 * tx) = w;
     }
+}
+
+// The score kernels alone (later head chunks), and the first chunk's beside the
+// key sort's segments (the first nseg workgroups, a multiple of 8 so that the
+// tiles keep their XCDs): the segments are a chain of dependent steps on a few
+// CUs, and the scores need neither them nor what follows from them (segments 23
+// us and scores 35 us one after the other, 45 us together, at 2 x 1,024 fp32 rows,
+// 8 heads).
+template <typename T, int D, int QF>
+__global__ void __launch_bounds__(256) dense_mfma_kernel(DnP p, SortTopArgs s, int nseg) {
+    extern __shared__ __align__(16) uint32_t dn_lds[];
+    if ((int)blockIdx.x < nseg)
+        sort_seg_blocks<uint16_t>(s.gkv, s.n, s.segs, s.segcount, s.perm, dn_lds, (int)blockIdx.x, nseg);
+    else
+        dense_mfma_tile<T, D, QF>(p, (int64_t)blockIdx.x - nseg);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) dense_valu_kernel(DnP p, SortTopArgs s, int nseg) {
+    extern __shared__ __align__(16) uint32_t dn_lds[];
+    if ((int)blockIdx.x < nseg)
+        sort_seg_blocks<uint16_t>(s.gkv, s.n, s.segs, s.segcount, s.perm, dn_lds, (int)blockIdx.x, nseg);
+    else
+        dense_valu_tile<T>(p, (int64_t)blockIdx.x - nseg, (float *)dn_lds);
 }
 
 // ---------------------------------------------------------------- select

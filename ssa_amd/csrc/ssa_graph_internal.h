@@ -28,6 +28,10 @@ struct SortTopArgs {
 };
 int ssa_sort_top_setup(const uint16_t *ids, int rows, int n, int P, int32_t *perm,
                        int32_t *bstart, int32_t *bsize, uint16_t *tmp, SortTopArgs *a);
+// the top levels alone, as set up (16-bit positions)
+int ssa_launch_sort_top(const SortTopArgs &a, hipStream_t st);
+// and the segment pass alone
+int ssa_launch_sort_seg(const SortTopArgs &a, hipStream_t st);
 // workgroups of the segment launch (SEG_WAVES waves each) for rows x n keys
 int ssa_sort_seg_blocks(int rows, int n);
 int ssa_launch_bucket_sort(const uint16_t *ids, int rows, int n, int P, int32_t *perm,

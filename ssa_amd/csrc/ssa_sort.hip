@@ -169,6 +169,19 @@ static int launch_sort(const uint16_t *ids, int rows, int n, int NB, int32_t *pe
     return launch_seg<Pos>(gkv, rows, n, segs, segcount, perm, st);
 }
 
+int ssa_launch_sort_top(const SortTopArgs &a, hipStream_t st) {
+    SSA_ALLOW_LDS((sort_top_kernel<uint16_t>), a.lds);
+    hipLaunchKernelGGL((sort_top_kernel<uint16_t>), dim3(a.rows), dim3(SORT_THREADS), a.lds, st, a.ids,
+                       a.n, a.NB, a.perm, a.bstart, a.bsize, a.gkv, a.segs, a.segcount, a.glb,
+                       a.tl_in_lds, a.cap);
+    SSA_CHECK_LAUNCH();
+    return SSA_OK;
+}
+
+int ssa_launch_sort_seg(const SortTopArgs &a, hipStream_t st) {
+    return launch_seg<uint16_t>(a.gkv, a.rows, a.n, a.segs, a.segcount, a.perm, st);
+}
+
 int ssa_launch_bucket_sort(const uint16_t *ids, int rows, int n, int P, int32_t *perm,
                            int32_t *bstart, int32_t *bsize, uint16_t *tmp, hipStream_t st,
                            bool counter_clear) {
