@@ -589,8 +589,8 @@ def gather_attention_fwd(q, k, v, neighbors, valid, scale, fp32w=False, dropout_
 def gather_attention_bwd(q, k, v, neighbors, valid, scale, fp32w, dropout_p, seed, dout,
                          deterministic=False):
     """dq, dk, dv (fp32).  deterministic: ssa_sparse_gather_attention_bwd_det,
-    whose dK / dV sums are fixed-point and so the same bits on every run (a
-    workspace is allocated here); else the fp32-atomic backward."""
+    whose dK / dV are the same bits on every run (a workspace is allocated
+    here); else the fp32-atomic backward."""
     check_apply_shapes(q, k, v, neighbors, valid, dout)
     require_device(q, k, v, neighbors, valid, dout)
     d = q.shape[-1]

@@ -6,21 +6,21 @@
 // 2 K d read-modify-writes of memory per query row (at 131,072 rows of 128
 // slots, d = 128, 8 kv heads of 4,096 keys: 4.3e9 fp32 atomics, 100 ms).  Here
 // the graph is transposed instead, and every key row is summed by one wavefront
-// in registers (times of that shape in bf16 behind each kernel; 1.4 ms in all):
+// in registers (times of that shape in bf16 behind each kernel; 1.33 ms in all):
 //
 //   1. grad_count_kernel   counts the slots of each key row per block of query
 //                          rows in LDS; the count before a slot is its rank
-//                          (48 us)
+//                          (47 us)
 //   2. grad_chunk_kernel,  prefixes over the blocks and over the key rows: the
 //      grad_list_kernel,   place of every slot in its key row's list, and the
 //      grad_segs_kernel    lists cut into segments of at most `seg` entries
-//                          (15 + 8 + 5 us)
+//                          (15 + 10 + 5 us)
 //   3. grad_rows_kernel    per query row: scores and dO.V, the softmax, dQ;
 //                          each slot's two weights go to its place in the list
-//                          (772 us)
-//   4. grad_keys_kernel    per segment: dK = sum draw q, dV = sum p' dO (483 us)
+//                          (756 us)
+//   4. grad_keys_kernel    per segment: dK = sum draw q, dV = sum p' dO (473 us)
 //   5. grad_join_kernel    key rows of several segments: sum of their partials
-//                          (22 us)
+//                          (21 us)
 //
 // Numerics: scores, softmax, weights and sums in fp32 as in the forward (16-bit
 // products are exact in fp32).  Deterministic mode: the order of a list's
@@ -342,7 +342,7 @@ struct RowOut {
 // One wavefront per query row, as in the forward: ids in LDS, K and V rows
 // gathered together for the scores and dO.V, the softmax per slot, then the K
 // rows again for dQ.  Bound: the gathers' L2 delivery (3 rows of d per slot
-// against the forward's 2: 12.9 GB in 772 us, 16.7 TB/s) and the VALU work of
+// against the forward's 2: 12.9 GB in 756 us, 17.0 TB/s) and the VALU work of
 // the products.
 template <typename T, typename TD, int D, int U, bool OFF32>
 __global__ void __launch_bounds__(WAVES * SSA_WAVE)
@@ -648,7 +648,7 @@ __global__ void __launch_bounds__(WAVES * SSA_WAVE) grad_bound_kernel(GradP gp) 
 
 // One wavefront per segment of a key row's list; RPI entries a step, U steps
 // in flight.  Bound: the L2 delivery of the q and dO rows (2 rows of d per
-// entry: 8.6 GB in 483 us, 17.8 TB/s) and their FMAs.
+// entry: 8.6 GB in 473 us, 18.2 TB/s) and their FMAs.
 template <typename T, typename TD, int D, int U, bool DET>
 __global__ void __launch_bounds__(WAVES * SSA_WAVE)
 grad_keys_kernel(GradP gp) {

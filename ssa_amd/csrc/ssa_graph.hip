@@ -40,6 +40,10 @@
 //                      (a tied kk-th score; in LSH mode any equal selected
 //                      scores) are rebuilt and run through an exact replay of
 //                      the reference's chunked nth_element + sort (:904-922).
+//
+// FULL-mode calls whose lists hold about as many members per query as there
+// are keys take steps 3 to 5 in the dense form instead (ssa_graph_dense.h; the
+// rule is dense_form below), with the same graph bit for bit.
 #include <stdarg.h>
 #include <stdio.h>
 
