@@ -339,6 +339,18 @@ struct RowOut {
     }
 };
 
+// A slot in LDS: the key id it attends to, or negative: masked (its id, whose row
+// is read and weighed 0 as autograd does), or no key at all (padding up to a
+// whole step, an id out of range), which takes nothing, whatever key row 0, read
+// in its place, holds.  OFF32 (ids below 2^24): the row is the low 24 bits, so
+// the address takes no step of its own.
+template <bool OFF32> struct SlotId {
+    static constexpr int32_t NONE = OFF32 ? (int32_t)0xc0000000 : INT32_MIN;
+    static __device__ __forceinline__ int32_t masked(int32_t y) { return OFF32 ? (y | INT32_MIN) : ~y; }
+    // the row read for a slot (not OFF32)
+    static __device__ __forceinline__ int32_t row(int32_t x) { return x >= 0 ? x : x == NONE ? 0 : ~x; }
+};
+
 // One wavefront per query row, as in the forward: ids in LDS, K and V rows
 // gathered together for the scores and dO.V, the softmax per slot, then the K
 // rows again for dQ.  Bound: the gathers' L2 delivery (3 rows of d per slot
@@ -362,7 +374,7 @@ grad_rows_kernel(GradP gp) {
     const int lane = lane_id();
     const int sub = lane / LPR, li = lane % LPR;
     const int Kp = (p.K + STEP - 1) / STEP * STEP;
-    // key ids; masked and padding slots hold INT_MIN (row 0)
+    using S = SlotId<OFF32>;
     int32_t *ix = reinterpret_cast<int32_t *>(smem) + (int64_t)wid * 3 * Kp;
     float *sc = reinterpret_cast<float *>(ix + Kp);      // scores, p, then draw
     float *dpv = sc + Kp;                                // dO.V per slot
@@ -388,13 +400,13 @@ grad_rows_kernel(GradP gp) {
         if constexpr (OFF32)
             return reinterpret_cast<const T *>((const char *)kb + (__umul24((uint32_t)x, krb) +
                                                                   (uint32_t)lofs * (uint32_t)sizeof(T)));
-        else return kb + (int64_t)(x < 0 ? 0 : x) * p.ksn + lofs;
+        else return kb + (int64_t)S::row(x) * p.ksn + lofs;
     };
     auto vrow = [&](int x) __attribute__((always_inline)) {
         if constexpr (OFF32)
             return reinterpret_cast<const T *>((const char *)vb + (__umul24((uint32_t)x, vrb) +
                                                                   (uint32_t)lofs * (uint32_t)sizeof(T)));
-        else return vb + (int64_t)(x < 0 ? 0 : x) * p.vsn + lofs;
+        else return vb + (int64_t)S::row(x) * p.vsn + lofs;
     };
 
     auto slots = [&](auto i32) __attribute__((always_inline)) {
@@ -405,8 +417,8 @@ grad_rows_kernel(GradP gp) {
             for (int u = 0; u < APPLY_SLOT_BATCH; ++u) {
                 const int j = j0 + u * SSA_WAVE + lane;
                 const int64_t y = rs.y[u];
-                const bool ok = j < p.K && !rs.marked(u) && y >= 0 && y < p.M;
-                if (j < Kp) ix[j] = ok ? (int)y : INT32_MIN;
+                const bool in = j < p.K && y >= 0 && y < p.M;
+                if (j < Kp) ix[j] = !in ? S::NONE : rs.marked(u) ? S::masked((int32_t)y) : (int32_t)y;
             }
         }
     };
@@ -490,6 +502,17 @@ grad_rows_kernel(GradP gp) {
         Raw<T, VEC> kv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) kv[u] = load_raw<T, VEC>(krow(xi[u]));
+        bool none = false;
+#pragma unroll
+        for (int u = 0; u < U; ++u) none |= xi[u] == S::NONE;
+        if (wave_ballot(none)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (xi[u] == S::NONE) {
+                    w[u] = 0.f;
+                    __builtin_memset(&kv[u], 0, sizeof(kv[u]));
+                }
+        }
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -578,11 +601,13 @@ grad_rows_long_kernel(GradP gp) {
         const float mask = mask_of(j);
         const float draw = pj * (R.dotv(dof, x) * mask - pdp) * p.scale;
         if (j < p.K && li == 0) ro.put(gp, x, j, draw, pj * mask);
-        const float w = j < p.K ? draw : 0.f;
+        // a masked slot's own row, weighed 0; none for padding and ids out of range
+        const int64_t y = j >= p.K ? -1 : p.nb32 ? (int64_t)p.nb32[row * p.K + j] : R.nb[j];
+        if (y < 0 || y >= p.M) continue;
         float kf[VEC];
-        load_vec<T, VEC>(R.kb + (int64_t)(x < 0 ? 0 : x) * p.ksn + R.lofs, kf);
+        load_vec<T, VEC>(R.kb + y * p.ksn + R.lofs, kf);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) dqa[e] = fmaf(w, kf[e], dqa[e]);
+        for (int e = 0; e < VEC; ++e) dqa[e] = fmaf(draw, kf[e], dqa[e]);
     }
 #pragma unroll
     for (int o = LPR; o < SSA_WAVE; o <<= 1)

@@ -210,3 +210,61 @@ def test_gradient_workspace_is_checked():
     assert b"workspace" in L.ssa_last_error()
     a.dk.dtype = _lib.SSA_F16
     assert L.ssa_sparse_gather_attention_grad_workspace_bytes(ctypes.byref(a)) < 0
+
+
+# ---- rows and slots that hold infinities, NaNs or nothing
+
+@pytest.mark.parametrize("K", [65, 3073], ids=["lds", "long"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_dq_takes_nothing_from_a_key_no_slot_names(K, dtype, bad):
+    """Key row 0 is named by no slot (K is no multiple of a step, some slots
+    are masked, some ids lie out of range): what it holds reaches no gradient,
+    bit for bit."""
+    from ssa_amd import _lib
+    N = 20 if K < 100 else 3
+    q, k, v, nb, va, dout = _inputs(2, 4, 2, N, 90, 64, K, dtype, 13)
+    nb.clamp_min_(1)
+    nb[:, :, ::2, 3], nb[:, :, ::3, 5] = -7, 90
+    graphs = {"int64": (nb, va), "int32": (torch.where(va, nb, -1).to(torch.int32), None)}
+    for name, (n, m) in graphs.items():
+        runs = []
+        for x in (1.0, bad):
+            k[:, :, 0] = x
+            runs.append(_lib.gather_attention_grad(q, k, v, n, m, 0.125, False, 0.0, 0, dout, True))
+        for a, b in zip(*runs):
+            assert torch.isfinite(a).all() and torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("K", [12, 3100], ids=["lds", "long"])
+@pytest.mark.parametrize("det", [False, True])
+def test_gradients_of_rows_without_any_key(K, det):
+    """Query rows whose ids all lie out of range (an int32 graph's -1) have no
+    key: their dq is zero, as the atomic backward leaves it."""
+    from ssa_amd import _lib
+    q, k, v, nb, va, dout = _inputs(1, 2, 1, 6, 50, 64, K, torch.float32, 8)
+    va[:] = True
+    nb[0, 1, 3] = -1
+    old = _lib.gather_attention_bwd(q, k, v, nb, va, 0.125, False, 0.0, 0, dout)
+    for n, m in ((nb, va), (nb.to(torch.int32), None)):
+        new = _lib.gather_attention_grad(q, k, v, n, m, 0.125, False, 0.0, 0, dout, det)
+        assert (new[0][0, 1, 3] == 0).all() and (old[0][0, 1, 3] == 0).all()
+        for name, a, b in zip(("dq", "dk", "dv"), new, old):
+            _check_grad_rows(name, a, b, torch.float32)
+
+
+@pytest.mark.parametrize("K", [12, 3100], ids=["lds", "long"])
+@pytest.mark.parametrize("det", [False, True])
+def test_dq_weighs_a_masked_slots_own_row(K, det):
+    """A masked slot's weight of 0 times its own key row, as autograd has it:
+    NaN in dq where that row is infinite, in no other query row."""
+    from ssa_amd import _lib
+    q, k, v, nb, va, dout = _inputs(1, 2, 1, 6, 50, 64, K, torch.float32, 8)
+    nb %= 40
+    nb[0, 1, 2, 4], va[0, 1, 2, 4] = 45, False
+    k[0, 0, 45] = float("inf")
+    old = _lib.gather_attention_bwd(q, k, v, nb, va, 0.125, False, 0.0, 0, dout)[0]
+    new = _lib.gather_attention_grad(q, k, v, nb, va, 0.125, False, 0.0, 0, dout, det)[0]
+    assert torch.equal(torch.isnan(new), torch.isnan(old))
+    rows = torch.isnan(new).all(-1)
+    assert rows[0, 1, 2] and rows.sum() == 1
