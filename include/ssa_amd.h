@@ -251,11 +251,13 @@ int ssa_sparse_gather_attention_bwd(const ssa_apply_bwd_args *a, void *stream);
  *   dk and dv (B,Hkv,M,d), all in q's type or all fp32, are WRITTEN.  Views with
  *   a unit last stride.  Sums in fp32, rounded once.
  *   deterministic: the same bits on every run (fp64 sums of terms rounded to a
- *   grid of the key row, exact in any order); a key row whose bound (slots x
- *   largest weight x largest |q| or |dout|) is not finite gets NaN.
+ *   grid of the key row, exact in any order); a key row whose bound (its slots x
+ *   the largest |weight| x largest |q| or |dout| of the row in a slot) is not
+ *   finite gets NaN.
  * Needs a 256-byte aligned workspace of
- * ssa_sparse_gather_attention_grad_workspace_bytes: about 20 bytes per slot of
- * as many (batch, kv head) groups as hold 2^28 slots (at least one). */
+ * ssa_sparse_gather_attention_grad_workspace_bytes: about 20 bytes per slot
+ * (24 when deterministic) of as many (batch, kv head) groups as hold 2^28
+ * slots (at least one). */
 typedef struct {
     ssa_apply_args fwd;
     ssa_tensor4 dout;

@@ -66,12 +66,12 @@ struct GradP {
     uint32_t *klen;        // (ng, M)
     int32_t *kfirst;       // (ng, M) first segment
     int2 *kpart;           // (ng, M) first partial, partials (0: none)
-    uint32_t *wmax;        // (ng, M, 2) largest |draw|, |p'| as float bits (deterministic)
+    uint32_t *bnd;         // (ng * gslots) each entry's term bounds, as row_bound packs them (deterministic)
+    uint32_t *wmax;        // (ng, M, 2) the largest of a key row's dK and dV bounds (deterministic)
     uint8_t *poison;       // (ng, M) 1: dK is NaN, 2: dV is NaN
     GradSeg *segs;         // (ng, segcap)
     int32_t *nseg;         // (ng)
     void *part;            // (ng * partcap, 2, d) float, or double when deterministic
-    uint32_t *xmax;        // {largest |q|, largest |dO|} as float bits (deterministic)
 };
 
 constexpr int CNT_THREADS = 1024;
@@ -302,6 +302,26 @@ __device__ __forceinline__ void store_grad(void *base, int64_t at, float v, bool
     else Cvt<T>::store((T *)base + at, v);
 }
 
+// Deterministic mode: at least |w| x xm, xm the largest finite or infinite |x| of
+// the row that w weighs, as a bf16 pattern (0: the term is 0; NaN above infinity).
+// A NaN element of x is in no bound: its term carries it.
+__device__ __forceinline__ uint32_t row_bound(float w, float xm) {
+    const float b = fabsf(w) * xm;
+    if (b != b) return w == 0.f ? 0u : 0x7fffu;
+    if (w == 0.f || xm == 0.f) return 0u;
+    const uint32_t up = (__float_as_uint(fmaxf(b, 1.17549435e-38f)) + 0xffffu) >> 16;
+    return b == INFINITY ? up : min(up, 0x7f7fu);     // rounded down at the top: grid_magic doubles it
+}
+
+// largest |x| over a row's lanes, NaN left out
+template <typename T, int VEC>
+__device__ __forceinline__ float row_absmax(const T (&x)[VEC]) {
+    float m = 0.f;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) m = fmaxf(m, fabsf(to_f32(x[e])));
+    return wave_max(m);
+}
+
 // What a row's slots leave for their key rows: per slot the weights of q (draw)
 // and of dO (p') at the slot's place in the key's list.  A masked slot has no
 // place; its weights are 0, or NaN in a row without a finite softmax, which
@@ -313,6 +333,7 @@ struct RowOut {
     int64_t ki;                // the group's first key row
     int64_t slot;              // the row's first slot in the graph
     uint32_t qoff, dooff;
+    float qm = 0.f, dm = 0.f;  // deterministic: the row's largest |q| and |dO|
     __device__ __forceinline__ RowOut(const GradP &p, int64_t row, int gl, int hl, int n) {
         const int64_t lrow = row - (int64_t)p.g0 * p.grows;
         const int c = (int)((lrow - (int64_t)gl * p.grows) / p.crows);
@@ -328,6 +349,7 @@ struct RowOut {
         if (x >= 0) {
             const int64_t at = kbegin[x] + tab[x] + rank[j];
             p.ent[at] = make_uint4(qoff, dooff, __float_as_uint(draw), __float_as_uint(pw));
+            if (p.bnd) p.bnd[at] = (row_bound(draw, qm) << 16) | row_bound(pw, dm);
         } else if (draw != draw || pw != pw) {
             const int64_t y = p.a.nb32 ? (int64_t)p.a.nb32[slot + j] : p.a.nb[slot + j];
             if (y >= 0 && y < p.a.M) {
@@ -475,7 +497,11 @@ grad_rows_kernel(GradP gp) {
         dpv[j] = dpj;
     }
     pdp = wave_sum(pdp);
-    const RowOut ro(gp, row, gl, h - g * p.rep, n);
+    RowOut ro(gp, row, gl, h - g * p.rep, n);
+    if (gp.bnd) {
+        ro.qm = row_absmax(qr.e);
+        ro.dm = row_absmax(dr.e);
+    }
     for (int j = lane; j < Kp; j += SSA_WAVE) {
         float draw = 0.f;
         if (j < p.K) {
@@ -590,7 +616,11 @@ grad_rows_long_kernel(GradP gp) {
         if (j < p.K && li == 0) pdp += pj * dpj;
     }
     pdp = wave_sum(pdp);
-    const RowOut ro(gp, row, gl, h - g * p.rep, n);
+    RowOut ro(gp, row, gl, h - g * p.rep, n);
+    if (gp.bnd) {
+        ro.qm = row_absmax(qf);
+        ro.dm = row_absmax(dof);
+    }
     float dqa[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) dqa[e] = 0.f;
@@ -621,21 +651,19 @@ grad_rows_long_kernel(GradP gp) {
 
 // ---------------------------------------------------------------- 4. key rows
 // The grid a key row's terms are rounded to in deterministic mode: 2^(e - 51)
-// for 2^e above count x largest weight x largest |x|.  A partial sum then
-// stays below 2^52 grid units (each term is off by at most half a unit), so
-// adding terms in fp64 is exact and the order does not matter.  Returned as
+// for 2^e above 2 x count x the largest bound of its terms (row_bound).  A partial
+// sum then stays below 2^52 grid units (each term is off by at most half a unit),
+// so adding terms in fp64 is exact and the order does not matter.  Returned as
 // the constant 1.5 x 2^52 units: adding and subtracting it rounds to the grid.
-// 0: no term; NaN: the bound is not finite.
-__device__ __forceinline__ double grid_magic(uint32_t cnt, float w, float x) {
-    const double bound = (double)cnt * (double)w * (double)x;
-    if (!(bound == bound) || bound > 1e300) return __builtin_nan("");
+// 0: no term but zeros (and NaNs); NaN: the bound is not finite.
+__device__ __forceinline__ double grid_magic(uint32_t cnt, uint32_t code) {
+    const double bound = 2.0 * (double)cnt * (double)__uint_as_float(code << 16);
+    if (!(bound < 1e300)) return __builtin_nan("");
     if (!(bound > 0.0)) return 0.0;
     int e = 0;
     (void)frexp(bound, &e);                 // bound < 2^e
     return ldexp(1.5, e + 1);
 }
-
-__device__ __forceinline__ uint32_t abs_bits(float v) { return __float_as_uint(v) & 0x7fffffffu; }
 
 // the segment of this wavefront, or nullptr past the group's last
 __device__ __forceinline__ const GradSeg *wave_segment(const GradP &gp, int &gl) {
@@ -649,8 +677,8 @@ __device__ __forceinline__ const GradSeg *wave_segment(const GradP &gp, int &gl)
     return gp.segs + (int64_t)gl * gp.segcap + si;
 }
 
-// deterministic mode: each key row's largest weights (integer maxima of float
-// bits, whose result does not depend on their order)
+// deterministic mode: the largest bounds of each key row's terms (integer maxima
+// of float patterns, whose result does not depend on their order)
 __global__ void __launch_bounds__(WAVES * SSA_WAVE) grad_bound_kernel(GradP gp) {
     int gl;
     const GradSeg *s = wave_segment(gp, gl);
@@ -658,9 +686,9 @@ __global__ void __launch_bounds__(WAVES * SSA_WAVE) grad_bound_kernel(GradP gp) 
     const GradSeg sg = *s;
     uint32_t wk = 0, wv = 0;
     for (int i = lane_id(); i < sg.len; i += SSA_WAVE) {
-        const uint4 e = gp.ent[sg.begin + i];
-        wk = max(wk, e.z & 0x7fffffffu);
-        wv = max(wv, e.w & 0x7fffffffu);
+        const uint32_t b = gp.bnd[sg.begin + i];
+        wk = max(wk, b >> 16);
+        wv = max(wv, b & 0xffffu);
     }
     wk = wave_max_u(wk);
     wv = wave_max_u(wv);
@@ -697,8 +725,8 @@ grad_keys_kernel(GradP gp) {
     double mk = 0.0, mv = 0.0;
     if constexpr (DET) {
         const uint32_t len = gp.klen[ki];
-        mk = grid_magic(len, __uint_as_float(gp.wmax[2 * ki]), __uint_as_float(gp.xmax[0]));
-        mv = grid_magic(len, __uint_as_float(gp.wmax[2 * ki + 1]), __uint_as_float(gp.xmax[1]));
+        mk = grid_magic(len, gp.wmax[2 * ki]);
+        mv = grid_magic(len, gp.wmax[2 * ki + 1]);
     }
 
     A ak[VEC], av[VEC];
@@ -821,48 +849,6 @@ __global__ void __launch_bounds__(WAVES * SSA_WAVE) grad_join_kernel(GradP gp) {
     }
 }
 
-// Largest |x| over the rows of a (B, H, N, d) view, as float bits
-// (deterministic mode): a lane group per row, a row's elements in pieces of
-// VEC, one atomic per workgroup.
-template <typename T, int D>
-__device__ __forceinline__ uint32_t rows_absmax(const T *x, int64_t sb, int64_t sh, int64_t sn, int H,
-                                                int N, int d, int64_t rows) {
-    using G = Geo<T, D>;
-    constexpr int VEC = G::VEC, LPR = G::LPR, RPB = 256 / LPR;
-    const int li = threadIdx.x % LPR;
-    uint32_t m = 0;
-    if (li * VEC < d) {
-        for (int64_t r = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR; r < rows;
-             r += (int64_t)gridDim.x * RPB) {
-            const uint32_t bh = (uint32_t)(r / N);
-            const Raw<T, VEC> v = load_raw<T, VEC>(x + (int64_t)(bh / (uint32_t)H) * sb +
-                                                   (int64_t)(bh % (uint32_t)H) * sh + (r - (int64_t)bh * N) * sn +
-                                                   li * VEC);
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) m = max(m, abs_bits(to_f32(v.e[e])));
-        }
-    }
-    return wave_max_u(m);
-}
-
-// workgroups alternate between q (xmax[0]) and dO (xmax[1])
-template <typename T, typename TD, int D>
-__global__ void __launch_bounds__(256) grad_absmax_kernel(GradP p) {
-    __shared__ uint32_t red[4];
-    const ApplyP &a = p.a;
-    const uint32_t m = blockIdx.y == 0
-        ? rows_absmax<T, D>((const T *)a.q, a.qsb, a.qsh, a.qsn, a.Hq, a.N, a.d, a.rows)
-        : rows_absmax<TD, D>((const TD *)p.dout, p.dosb, p.dosh, p.dosn, a.Hq, a.N, a.d, a.rows);
-    if (lane_id() == 0) red[threadIdx.x / SSA_WAVE] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicMax(&p.xmax[blockIdx.y], max(max(red[0], red[1]), max(red[2], red[3])));
-}
-
-__global__ void __launch_bounds__(256) grad_zero_kernel(uint32_t *w, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
-        w[i] = 0u;
-}
-
 // zeros over a (B, H, N, d) view (no query row or no slot reaches anything)
 template <typename T>
 __global__ void __launch_bounds__(256) grad_fill0_kernel(void *out, int64_t sb, int64_t sh, int64_t sn,
@@ -881,7 +867,7 @@ constexpr int64_t GRAD_SLOTS = (int64_t)1 << 28;   // slots per launch: 5.4 GB o
 int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
 struct GradLayout {
-    int64_t ent, rank, tab, kbegin, klen, kfirst, kpart, wmax, poison, segs, nseg, part, xmax, total;
+    int64_t ent, rank, tab, kbegin, klen, kfirst, kpart, bnd, wmax, poison, segs, nseg, part, total;
 };
 
 // Sizes of one launch over `ng` groups (whole (b, kv head) groups, so no key
@@ -910,12 +896,12 @@ GradLayout grad_plan(GradP &p, int det) {
     L.klen = take(keys * 4);
     L.kfirst = take(keys * 4);
     L.kpart = take(keys * 8);
+    L.bnd = take(det ? slots * 4 : 0);
     L.wmax = take(det ? keys * 8 : 0);
     L.poison = take(keys + 4);
     L.segs = take((int64_t)p.ng * p.segcap * (int64_t)sizeof(GradSeg));
     L.nseg = take((int64_t)p.ng * 4);
     L.part = take((int64_t)p.ng * p.partcap * 2 * p.a.d * (det ? 8 : 4));
-    L.xmax = take(8);
     L.total = o;
     return L;
 }
@@ -961,20 +947,13 @@ int launch_grad(GradP p, int det, char *ws, hipStream_t st) {
     p.klen = (uint32_t *)(ws + L.klen);
     p.kfirst = (int32_t *)(ws + L.kfirst);
     p.kpart = (int2 *)(ws + L.kpart);
+    p.bnd = det ? (uint32_t *)(ws + L.bnd) : nullptr;
     p.wmax = det ? (uint32_t *)(ws + L.wmax) : nullptr;
     p.poison = (uint8_t *)(ws + L.poison);
     p.segs = (GradSeg *)(ws + L.segs);
     p.nseg = (int32_t *)(ws + L.nseg);
     p.part = ws + L.part;
-    p.xmax = (uint32_t *)(ws + L.xmax);
     const ApplyP &a = p.a;
-    if (det) {
-        hipLaunchKernelGGL(grad_zero_kernel, dim3(1), dim3(256), 0, st, p.xmax, (int64_t)2);
-        SSA_CHECK_LAUNCH();
-        const unsigned gr = (unsigned)std::min<int64_t>(ceil_div(a.rows, 256), 256);
-        hipLaunchKernelGGL((grad_absmax_kernel<T, TD, D>), dim3(gr, 2), dim3(256), 0, st, p);
-        SSA_CHECK_LAUNCH();
-    }
     const size_t clds = (size_t)std::min(a.M, CNT_KEYS) * 4;
     for (int g0 = 0; g0 < all; g0 += per) {
         p.g0 = g0;
