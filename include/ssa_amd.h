@@ -250,8 +250,8 @@ int ssa_sparse_gather_attention_bwd(const ssa_apply_bwd_args *a, void *stream);
  *   valid, or neighbors32); dout (B,Hq,N,d) in q's type or fp32; dq (B,Hq,N,d),
  *   dk and dv (B,Hkv,M,d), all in q's type or all fp32, are WRITTEN.  Views with
  *   a unit last stride.  Sums in fp32, rounded once.
- *   deterministic: the same bits on every run (fp64 sums of terms rounded to a
- *   grid of the key row, exact in any order); a key row whose bound (its slots x
+ *   deterministic: the same bits on every run (fp64 sums of terms rounded to two
+ *   grids of the key row, exact in any order); a key row whose bound (its slots x
  *   the largest |weight| x largest |q| or |dout| of the row in a slot) is not
  *   finite gets NaN.
  * Needs a 256-byte aligned workspace of

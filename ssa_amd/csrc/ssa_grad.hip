@@ -26,7 +26,9 @@
 // products are exact in fp32).  Deterministic mode: the order of a list's
 // entries varies between runs, so its sums are made independent of the order:
 // each term (exact in fp64) is rounded to a grid of its key row coarse enough
-// that every partial sum is exact in fp64.
+// that every partial sum is exact in fp64, and what the rounding left to a
+// second, finer grid in a second sum, which keeps the bits of terms far below
+// the key row's largest (one huge element of a row that names the key).
 #include <algorithm>
 
 #include "ssa_apply_dev.h"
@@ -71,7 +73,7 @@ struct GradP {
     uint8_t *poison;       // (ng, M) 1: dK is NaN, 2: dV is NaN
     GradSeg *segs;         // (ng, segcap)
     int32_t *nseg;         // (ng)
-    void *part;            // (ng * partcap, 2, d) float, or double when deterministic
+    void *part;            // (ng * partcap, 2, d) float, or (.., 4, d) double when deterministic
 };
 
 constexpr int CNT_THREADS = 1024;
@@ -650,20 +652,42 @@ grad_rows_long_kernel(GradP gp) {
 }
 
 // ---------------------------------------------------------------- 4. key rows
-// The grid a key row's terms are rounded to in deterministic mode: 2^(e - 51)
-// for 2^e above 2 x count x the largest bound of its terms (row_bound).  A partial
-// sum then stays below 2^52 grid units (each term is off by at most half a unit),
-// so adding terms in fp64 is exact and the order does not matter.  Returned as
-// the constant 1.5 x 2^52 units: adding and subtracting it rounds to the grid.
-// 0: no term but zeros (and NaNs); NaN: the bound is not finite.
-__device__ __forceinline__ double grid_magic(uint32_t cnt, uint32_t code) {
-    const double bound = 2.0 * (double)cnt * (double)__uint_as_float(code << 16);
-    if (!(bound < 1e300)) return __builtin_nan("");
-    if (!(bound > 0.0)) return 0.0;
-    int e = 0;
-    (void)frexp(bound, &e);                 // bound < 2^e
-    return ldexp(1.5, e + 1);
-}
+// The grids a key row's terms are rounded to in deterministic mode: 2^(e - 51)
+// for 2^e above 2 x count x the largest bound of its terms (row_bound), and for
+// what that rounding leaves, at most half a unit a term, 2^(f - 51) for 2^f above
+// count x 2^(e - 51).  A partial sum then stays below 2^52 units of its grid, so
+// adding in fp64 is exact and the order does not matter.  Held as the constants
+// 1.5 x 2^52 units (0: no term but zeros and NaNs; NaN: the bound is not finite).
+// The first sum starts there, so adding a product rounds it to the grid; which way
+// half a unit goes depends on the sum, but then what is left is half a unit too and
+// on the second grid, whose rounding knows nothing of the sums: the two sums
+// together are the same in any order.
+struct GridSum {
+    double m1, m2, u2;     // u2: the second grid's unit
+    __device__ __forceinline__ GridSum(uint32_t cnt, uint32_t code) {
+        const double bound = 2.0 * (double)cnt * (double)__uint_as_float(code << 16);
+        m1 = m2 = u2 = 0.0;
+        if (!(bound < 1e300)) {
+            m1 = __builtin_nan("");
+        } else if (bound > 0.0) {
+            int e = 0, f = 0;
+            (void)frexp(bound, &e);                              // bound < 2^e
+            (void)frexp(ldexp((double)cnt, e - 51), &f);
+            m1 = ldexp(1.5, e + 1);
+            m2 = ldexp(1.5, f + 1);
+            u2 = ldexp(1.0, f - 51);
+        }
+    }
+    // hi from m1 on, lo from 0: its units, and m2's bits once a term
+    __device__ __forceinline__ void add(double w, double x, double &hi, uint64_t &lo) const {
+        const double s = fma(w, x, hi);
+        lo += (uint64_t)__double_as_longlong(fma(w, x, hi - s) + m2);
+        hi = s;
+    }
+    __device__ __forceinline__ double second(uint64_t lo, int terms) const {
+        return (double)(int64_t)(lo - (uint64_t)terms * (uint64_t)__double_as_longlong(m2)) * u2;
+    }
+};
 
 // the segment of this wavefront, or nullptr past the group's last
 __device__ __forceinline__ const GradSeg *wave_segment(const GradP &gp, int &gl) {
@@ -701,7 +725,9 @@ __global__ void __launch_bounds__(WAVES * SSA_WAVE) grad_bound_kernel(GradP gp) 
 
 // One wavefront per segment of a key row's list; RPI entries a step, U steps
 // in flight.  Bound: the L2 delivery of the q and dO rows (2 rows of d per
-// entry: 8.6 GB in 473 us, 18.2 TB/s) and their FMAs.
+// entry: 8.6 GB in 473 us, 18.2 TB/s) and their FMAs.  Deterministic: fp64 issue
+// and registers (1.27 M entries of d = 80: 114 us; 85 with one grid; four entries a
+// lane in flight instead of two leave 2 waves a SIMD, 126 us; one, 124 us).
 template <typename T, typename TD, int D, int U, bool DET>
 __global__ void __launch_bounds__(WAVES * SSA_WAVE)
 grad_keys_kernel(GradP gp) {
@@ -722,16 +748,16 @@ grad_keys_kernel(GradP gp) {
     const TD *db = (const TD *)gp.dout + b * gp.dosb + (int64_t)g * p.rep * gp.dosh + lofs;
     const int64_t ki = (int64_t)gl * p.M + sg.key;
 
-    double mk = 0.0, mv = 0.0;
-    if constexpr (DET) {
-        const uint32_t len = gp.klen[ki];
-        mk = grid_magic(len, gp.wmax[2 * ki]);
-        mv = grid_magic(len, gp.wmax[2 * ki + 1]);
-    }
+    const uint32_t cnt = DET ? gp.klen[ki] : 0u;
+    const GridSum sk(cnt, DET ? gp.wmax[2 * ki] : 0u), sv(cnt, DET ? gp.wmax[2 * ki + 1] : 0u);
 
     A ak[VEC], av[VEC];
+    constexpr int LV = DET ? VEC : 1;      // the second grids' sums
+    uint64_t nk[LV], nv[LV];
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) { ak[e] = (A)0; av[e] = (A)0; }
+    for (int e = 0; e < VEC; ++e) { ak[e] = DET ? (A)sk.m1 : (A)0; av[e] = DET ? (A)sv.m1 : (A)0; }
+#pragma unroll
+    for (int e = 0; e < LV; ++e) { nk[e] = 0; nv[e] = 0; }
     auto fetch = [&](int j0, uint4 (&en)[U]) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -770,13 +796,24 @@ grad_keys_kernel(GradP gp) {
             for (int e = 0; e < VEC; ++e) {
                 const float x = to_f32(qr[u].e[e]), y = to_f32(dr[u].e[e]);
                 if constexpr (DET) {
-                    ak[e] += ((double)wk[u] * (double)x + mk) - mk;
-                    av[e] += ((double)wv[u] * (double)y + mv) - mv;
+                    sk.add(wk[u], x, ak[e], nk[e]);
+                    sv.add(wv[u], y, av[e], nv[e]);
                 } else {
                     ak[e] = fmaf(wk[u], x, ak[e]);
                     av[e] = fmaf(wv[u], y, av[e]);
                 }
             }
+    }
+    A lk[LV], lv[LV];
+    if constexpr (DET) {
+        const int terms = (sg.len + STEP - 1) / STEP * U;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            ak[e] -= sk.m1;
+            av[e] -= sv.m1;
+            lk[e] = sk.second(nk[e], terms);
+            lv[e] = sv.second(nv[e], terms);
+        }
     }
 #pragma unroll
     for (int o = LPR; o < SSA_WAVE; o <<= 1)
@@ -784,17 +821,25 @@ grad_keys_kernel(GradP gp) {
         for (int e = 0; e < VEC; ++e) {
             ak[e] += __shfl_xor(ak[e], o, SSA_WAVE);
             av[e] += __shfl_xor(av[e], o, SSA_WAVE);
+            if constexpr (DET) {
+                lk[e] += __shfl_xor(lk[e], o, SSA_WAVE);
+                lv[e] += __shfl_xor(lv[e], o, SSA_WAVE);
+            }
         }
     if (sub != 0 || !live) return;
-    if constexpr (DET) {
-        if (mk != mk) for (int e = 0; e < VEC; ++e) ak[e] = mk;
-        if (mv != mv) for (int e = 0; e < VEC; ++e) av[e] = mv;
-    }
     if (sg.part >= 0) {
-        A *pa = (A *)gp.part + (int64_t)sg.part * 2 * p.d + lofs;
+        A *pa = (A *)gp.part + (int64_t)sg.part * (DET ? 4 : 2) * p.d + lofs;
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) { pa[e] = ak[e]; pa[p.d + e] = av[e]; }
+        for (int e = 0; e < VEC; ++e) {
+            pa[e] = ak[e];
+            pa[p.d + e] = av[e];
+            if constexpr (DET) { pa[2 * p.d + e] = lk[e]; pa[3 * p.d + e] = lv[e]; }
+        }
         return;
+    }
+    if constexpr (DET) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) { ak[e] += lk[e]; av[e] += lv[e]; }
     }
     const uint8_t f = gp.poison[ki];
     const int64_t ok = b * gp.dksb + g * gp.dksh + (int64_t)sg.key * gp.dksn + lofs;
@@ -827,17 +872,22 @@ __global__ void __launch_bounds__(WAVES * SSA_WAVE) grad_join_kernel(GradP gp) {
     const uint8_t f = gp.poison[ki];
     const int64_t gl = ki / p.M, x = ki % p.M;
     const int64_t grp = gp.g0 + gl, b = grp / p.Hkv, g = grp % p.Hkv;
-    const int d2 = 2 * p.d;
-    for (int i = lane_id(); i < d2; i += SSA_WAVE) {
-        const A *pa = (const A *)gp.part + (int64_t)kp.x * d2 + i;
+    const int d2 = 2 * p.d, pd = DET ? 2 * d2 : d2;
+    auto total = [&](const A *pa) __attribute__((always_inline)) {
         A sum = (A)0;
         for (int s0 = 0; s0 < kp.y; s0 += 8) {
             A v[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = s0 + u < kp.y ? pa[(int64_t)(s0 + u) * d2] : (A)0;
+            for (int u = 0; u < 8; ++u) v[u] = s0 + u < kp.y ? pa[(int64_t)(s0 + u) * pd] : (A)0;
 #pragma unroll
             for (int u = 0; u < 8; ++u) sum += v[u];
         }
+        return sum;
+    };
+    for (int i = lane_id(); i < d2; i += SSA_WAVE) {
+        const A *pa = (const A *)gp.part + (int64_t)kp.x * pd + i;
+        A sum = total(pa);
+        if constexpr (DET) sum += total(pa + d2);
         const bool isv = i >= p.d;
         const int e = isv ? i - p.d : i;
         float r = (f & (isv ? 2 : 1)) ? __builtin_nanf("") : (float)sum;
@@ -901,7 +951,7 @@ GradLayout grad_plan(GradP &p, int det) {
     L.poison = take(keys + 4);
     L.segs = take((int64_t)p.ng * p.segcap * (int64_t)sizeof(GradSeg));
     L.nseg = take((int64_t)p.ng * 4);
-    L.part = take((int64_t)p.ng * p.partcap * 2 * p.a.d * (det ? 8 : 4));
+    L.part = take((int64_t)p.ng * p.partcap * 2 * p.a.d * (det ? 16 : 4));
     L.total = o;
     return L;
 }
@@ -984,7 +1034,7 @@ int launch_grad(GradP p, int det, char *ws, hipStream_t st) {
         if (det) {
             hipLaunchKernelGGL(grad_bound_kernel, dim3(kgrid), dim3(WAVES * SSA_WAVE), 0, st, p);
             SSA_CHECK_LAUNCH();
-            hipLaunchKernelGGL((grad_keys_kernel<T, TD, D, UK, true>), dim3(kgrid),
+            hipLaunchKernelGGL((grad_keys_kernel<T, TD, D, 2, true>), dim3(kgrid),
                                dim3(WAVES * SSA_WAVE), 0, st, p);
             SSA_CHECK_LAUNCH();
             hipLaunchKernelGGL((grad_join_kernel<T, true>), dim3(jgrid), dim3(WAVES * SSA_WAVE), 0, st, p);

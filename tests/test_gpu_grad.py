@@ -307,3 +307,21 @@ def test_deterministic_key_rows_ignore_outliers_they_are_not_named_by(dtype, siz
     got = _lib.gather_attention_grad(q, *args, dout, True)
     for a, b in zip(got[1:], base[1:]):
         assert torch.equal(a[:, :, 8:], b[:, :, 8:])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("size", [1e6, 1e10, 1e14])
+def test_deterministic_sums_keep_their_bits_beside_an_outlier(dtype, size):
+    """One element of one dout row many orders above everything else: the
+    other elements of the key rows it reaches are as close to float64 as
+    without it.  Bar per element: BAR of the sum of the terms' sizes."""
+    from ssa_amd import _lib
+    q, k, v, nb, va, dout = _inputs(1, 2, 1, 200, 6, 64, 40, dtype, 23)
+    dout[0, 0, 9, 3] = size
+    scale = 0.125
+    dv = _lib.gather_attention_grad(q, k, v, nb, va, scale, False, 0.0, 0, dout, True)[2]
+    exp, absum = (t[2] for t in _reference(q, k, v, nb, va, scale, dout))
+    keep = torch.arange(64, device=DEV) != 3
+    err = ((dv.double() - exp).abs() / absum)[..., keep].max().item()
+    print(f"  outlier {size:.0e}: {err:.2e}", flush=True)
+    assert err <= BAR[dtype]
