@@ -255,9 +255,12 @@ int ssa_sparse_gather_attention_bwd(const ssa_apply_bwd_args *a, void *stream);
  *   the largest |weight| x largest |q| or |dout| of the row in a slot) is not
  *   finite gets NaN.
  * Needs a 256-byte aligned workspace of
- * ssa_sparse_gather_attention_grad_workspace_bytes: about 20 bytes per slot
- * (24 when deterministic) of as many (batch, kv head) groups as hold 2^28
- * slots (at least one). */
+ * ssa_sparse_gather_attention_grad_workspace_bytes: about 20 bytes per slot (24
+ * when deterministic), 61 (69) per key row, up to 2 per slot for a table and
+ * 16 d (64 d) per 256 to 4,096 slots, of as many (batch, kv head) groups as hold
+ * 2^28 slots and 2^25 key rows.  A group of more slots goes in parts of its query
+ * rows, whose sums are kept between them in 8 d (16 d) bytes per key row; one of
+ * more key rows takes what its rows need. */
 typedef struct {
     ssa_apply_args fwd;
     ssa_tensor4 dout;

@@ -53,9 +53,12 @@ struct GradP {
     int32_t out32;         // gradients are fp32 (else q's type)
     int32_t accumulate;    // dk, dv are added to (fp32 only)
     int32_t shift;         // entries hold row offsets in units of 1 << shift elements
-    // groups (b, kv head) of this launch: [g0, g0 + ng); rows per group, slots per group
+    // groups (b, kv head) of this launch: [g0, g0 + ng), with all their query rows,
+    // or one group's rows from r0 on (a part: the first, the last, or between)
     int32_t g0, ng;
-    int64_t grows, gslots;
+    int32_t first, last;
+    int64_t r0, row0;      // first row within its group, and of all
+    int64_t grows, gslots; // rows and slots of each group in this launch
     // blocks of `crows` query rows, nc of them per group
     int32_t crows, nc;
     int32_t seg;           // entries per segment
@@ -71,10 +74,19 @@ struct GradP {
     uint32_t *bnd;         // (ng * gslots) each entry's term bounds, as row_bound packs them (deterministic)
     uint32_t *wmax;        // (ng, M, 2) the largest of a key row's dK and dV bounds (deterministic)
     uint8_t *poison;       // (ng, M) 1: dK is NaN, 2: dV is NaN
+    void *acc;             // (M, 2, d) sums of a group's parts so far, float or double
     GradSeg *segs;         // (ng, segcap)
     int32_t *nseg;         // (ng)
     void *part;            // (ng * partcap, 2, d) float, or (.., 4, d) double when deterministic
 };
+
+// Workgroup of a launch: grids of more than GRID_X workgroups continue in y (the
+// runtime takes fewer than 2^32 threads in x).
+constexpr int64_t GRID_X = (int64_t)1 << 20;
+__device__ __forceinline__ int64_t launch_block() { return (int64_t)blockIdx.y * gridDim.x + blockIdx.x; }
+dim3 launch_grid(int64_t blocks) {
+    return blocks <= GRID_X ? dim3((unsigned)blocks) : dim3((unsigned)GRID_X, (unsigned)ceil_div(blocks, GRID_X));
+}
 
 constexpr int CNT_THREADS = 1024;
 constexpr int CNT_KEYS = 16384;        // key rows counted at a time: 64 KB of LDS
@@ -92,11 +104,13 @@ __device__ __forceinline__ int slot_key(const ApplyP &p, int64_t s) {
 // atomic per slot (a row's keys differ, so a wave's 64 atomics rarely meet).
 __global__ void __launch_bounds__(CNT_THREADS) grad_count_kernel(GradP p) {
     extern __shared__ uint32_t cnt[];
-    const int c = blockIdx.x % p.nc, gl = blockIdx.x / p.nc;
+    const int64_t blk = launch_block();
+    const int c = (int)(blk % p.nc), gl = (int)(blk / p.nc);
+    if (gl >= p.ng) return;
     const int64_t r0 = (int64_t)c * p.crows;
     const int64_t r1 = r0 + p.crows < p.grows ? r0 + p.crows : p.grows;
     const int64_t s0 = ((int64_t)gl * p.grows + r0) * p.a.K, s1 = ((int64_t)gl * p.grows + r1) * p.a.K;
-    const int64_t base = (int64_t)p.g0 * p.gslots;      // the graph's first slot of this launch
+    const int64_t base = p.row0 * p.a.K;                // the graph's first slot of this launch
     for (int k0 = 0; k0 < p.a.M; k0 += CNT_KEYS) {
         const int nk = p.a.M - k0 < CNT_KEYS ? p.a.M - k0 : CNT_KEYS;
         for (int i = threadIdx.x; i < nk; i += CNT_THREADS) cnt[i] = 0u;
@@ -115,7 +129,7 @@ __global__ void __launch_bounds__(CNT_THREADS) grad_count_kernel(GradP p) {
 // ---------------------------------------------------------------- 2. places
 // thread per (group, key row): prefix over the group's blocks
 __global__ void __launch_bounds__(256) grad_chunk_kernel(GradP p) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t i = launch_block() * 256 + threadIdx.x;
     if (i >= (int64_t)p.ng * p.a.M) return;
     const int64_t gl = i / p.a.M, x = i % p.a.M;
     uint32_t *t = p.tab + gl * p.nc * p.a.M + x;
@@ -155,7 +169,8 @@ constexpr int LIST_KEYS = 8;
 __global__ void __launch_bounds__(1024) grad_list_kernel(GradP p) {
     __shared__ int64_t wl[16];
     __shared__ int32_t ws[16], wp[16];
-    const int gl = blockIdx.x, tid = threadIdx.x, lane = lane_id(), wid = tid / SSA_WAVE;
+    const int gl = (int)launch_block(), tid = threadIdx.x, lane = lane_id(), wid = tid / SSA_WAVE;
+    if (gl >= p.ng) return;
     int64_t cl = (int64_t)gl * p.gslots;        // entries before this tile
     int32_t cs = 0, cp = 0;                     // segments, partials before it
     for (int k0 = 0; k0 < p.a.M; k0 += 1024 * LIST_KEYS) {
@@ -202,7 +217,7 @@ __global__ void __launch_bounds__(1024) grad_list_kernel(GradP p) {
 
 // thread per (group, key row): its segments
 __global__ void __launch_bounds__(256) grad_segs_kernel(GradP p) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t i = launch_block() * 256 + threadIdx.x;
     if (i >= (int64_t)p.ng * p.a.M) return;
     const int64_t gl = i / p.a.M;
     const uint32_t len = p.klen[i];
@@ -337,7 +352,7 @@ struct RowOut {
     uint32_t qoff, dooff;
     float qm = 0.f, dm = 0.f;  // deterministic: the row's largest |q| and |dO|
     __device__ __forceinline__ RowOut(const GradP &p, int64_t row, int gl, int hl, int n) {
-        const int64_t lrow = row - (int64_t)p.g0 * p.grows;
+        const int64_t lrow = row - p.row0;
         const int c = (int)((lrow - (int64_t)gl * p.grows) / p.crows);
         ki = (int64_t)gl * p.a.M;
         kbegin = p.kbegin + ki;
@@ -388,12 +403,12 @@ grad_rows_kernel(GradP gp) {
     const ApplyP &p = gp.a;
     extern __shared__ float smem[];
     const int64_t nblocks = ceil_div((int64_t)gp.ng * gp.grows, WAVES);
-    const int64_t blk = xcd_logical_block(blockIdx.x, nblocks);
+    const int64_t blk = xcd_logical_block(launch_block(), nblocks);
     if (blk >= nblocks) return;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / SSA_WAVE);
     const int64_t lrow = blk * WAVES + wid;
     if (lrow >= (int64_t)gp.ng * gp.grows) return;
-    const int64_t row = (int64_t)gp.g0 * gp.grows + lrow;
+    const int64_t row = gp.row0 + lrow;
     const int gl = (int)(lrow / gp.grows);
     const int lane = lane_id();
     const int sub = lane / LPR, li = lane % LPR;
@@ -566,12 +581,12 @@ grad_rows_long_kernel(GradP gp) {
     constexpr int VEC = G::VEC, LPR = G::LPR, RPI = G::RPI;
     const ApplyP &p = gp.a;
     const int64_t nblocks = ceil_div((int64_t)gp.ng * gp.grows, WAVES);
-    const int64_t blk = xcd_logical_block(blockIdx.x, nblocks);
+    const int64_t blk = xcd_logical_block(launch_block(), nblocks);
     if (blk >= nblocks) return;
     const int wid = threadIdx.x / SSA_WAVE;
     const int64_t lrow = blk * WAVES + wid;
     if (lrow >= (int64_t)gp.ng * gp.grows) return;
-    const int64_t row = (int64_t)gp.g0 * gp.grows + lrow;
+    const int64_t row = gp.row0 + lrow;
     const int gl = (int)(lrow / gp.grows);
     const int lane = lane_id();
     const int sub = lane / LPR, li = lane % LPR;
@@ -693,7 +708,7 @@ struct GridSum {
 __device__ __forceinline__ const GradSeg *wave_segment(const GradP &gp, int &gl) {
     const int64_t gblocks = ceil_div(gp.segcap, WAVES);
     const int64_t nblocks = gblocks * gp.ng;
-    const int64_t blk = xcd_logical_block(blockIdx.x, nblocks);
+    const int64_t blk = xcd_logical_block(launch_block(), nblocks);
     if (blk >= nblocks) return nullptr;
     gl = (int)(blk / gblocks);
     const int64_t si = (blk - gl * gblocks) * WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x / SSA_WAVE);
@@ -721,6 +736,15 @@ __global__ void __launch_bounds__(WAVES * SSA_WAVE) grad_bound_kernel(GradP gp) 
         atomicMax(w, wk);
         atomicMax(w + 1, wv);
     }
+}
+
+// The sum of a group's parts up to this one (a launch with all its rows: this
+// launch's), in the order of the parts; kept for the next unless this is the last.
+template <typename A>
+__device__ __forceinline__ A add_part(const GradP &gp, A *acc, A sum) {
+    if (!gp.first) sum += *acc;
+    if (!gp.last) *acc = sum;
+    return sum;
 }
 
 // One wavefront per segment of a key row's list; RPI entries a step, U steps
@@ -844,16 +868,20 @@ grad_keys_kernel(GradP gp) {
     const uint8_t f = gp.poison[ki];
     const int64_t ok = b * gp.dksb + g * gp.dksh + (int64_t)sg.key * gp.dksn + lofs;
     const int64_t ov = b * gp.dvsb + g * gp.dvsh + (int64_t)sg.key * gp.dvsn + lofs;
+    A *acc = (A *)gp.acc + (int64_t)sg.key * 2 * p.d + lofs;
     float x[VEC], y[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
-        x[e] = (f & 1) ? __builtin_nanf("") : (float)ak[e];
-        y[e] = (f & 2) ? __builtin_nanf("") : (float)av[e];
-        if (gp.accumulate) {
+        const A k = add_part(gp, acc + e, (f & 1) ? (A)__builtin_nanf("") : ak[e]);
+        const A v = add_part(gp, acc + p.d + e, (f & 2) ? (A)__builtin_nanf("") : av[e]);
+        x[e] = (float)k;
+        y[e] = (float)v;
+        if (gp.accumulate && gp.last) {
             x[e] += ((const float *)gp.dk)[ok + e];
             y[e] += ((const float *)gp.dv)[ov + e];
         }
     }
+    if (!gp.last) return;
     store_vec<T, VEC>(gp.dk, ok, x, gp.out32);
     store_vec<T, VEC>(gp.dv, ov, y, gp.out32);
 }
@@ -865,7 +893,7 @@ template <typename T, bool DET>
 __global__ void __launch_bounds__(WAVES * SSA_WAVE) grad_join_kernel(GradP gp) {
     using A = typename std::conditional<DET, double, float>::type;
     const ApplyP &p = gp.a;
-    const int64_t ki = (int64_t)blockIdx.x * WAVES + threadIdx.x / SSA_WAVE;
+    const int64_t ki = launch_block() * WAVES + threadIdx.x / SSA_WAVE;
     if (ki >= (int64_t)gp.ng * p.M) return;
     const int2 kp = gp.kpart[ki];
     if (kp.y == 0) return;
@@ -890,7 +918,9 @@ __global__ void __launch_bounds__(WAVES * SSA_WAVE) grad_join_kernel(GradP gp) {
         if constexpr (DET) sum += total(pa + d2);
         const bool isv = i >= p.d;
         const int e = isv ? i - p.d : i;
-        float r = (f & (isv ? 2 : 1)) ? __builtin_nanf("") : (float)sum;
+        float r = (float)add_part(gp, (A *)gp.acc + x * d2 + i,
+                                  (f & (isv ? 2 : 1)) ? (A)__builtin_nanf("") : sum);
+        if (!gp.last) continue;
         void *out = isv ? gp.dv : gp.dk;
         const int64_t at = isv ? b * gp.dvsb + g * gp.dvsh + x * gp.dvsn + e
                                : b * gp.dksb + g * gp.dksh + x * gp.dksn + e;
@@ -913,15 +943,26 @@ __global__ void __launch_bounds__(256) grad_fill0_kernel(void *out, int64_t sb, 
 
 // ---------------------------------------------------------------- launches
 constexpr int64_t GRAD_SLOTS = (int64_t)1 << 28;   // slots per launch: 5.4 GB of workspace
+constexpr int64_t GRAD_KEYS = (int64_t)1 << 25;    // key rows per launch: 2 GB
 
 int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
 struct GradLayout {
-    int64_t ent, rank, tab, kbegin, klen, kfirst, kpart, bnd, wmax, poison, segs, nseg, part, total;
+    int64_t ent, rank, tab, kbegin, klen, kfirst, kpart, bnd, wmax, poison, segs, nseg, part, acc, total;
 };
 
-// Sizes of one launch over `ng` groups (whole (b, kv head) groups, so no key
-// row's sum spans launches), and the workspace they take.
+// Groups and rows of each in one launch: whole (b, kv head) groups, so that few key
+// rows' sums span launches, as many as hold GRAD_SLOTS slots and GRAD_KEYS key rows;
+// of a group with more slots, the rows that hold GRAD_SLOTS.
+void grad_launches(GradP &p) {
+    const int64_t all = (int64_t)p.a.B * p.a.Hkv, rows = (int64_t)p.a.rep * p.a.N;
+    const int64_t K = std::max(p.a.K, 1), slots = std::max<int64_t>(rows * K, 1);
+    p.ng = (int)std::max<int64_t>(1, std::min(all, std::min(GRAD_SLOTS / slots, GRAD_KEYS / p.a.M)));
+    p.grows = std::min(rows, std::max<int64_t>(1, GRAD_SLOTS / K));
+    p.gslots = p.grows * p.a.K;
+}
+
+// Sizes of one launch over `ng` groups of `grows` rows, and the workspace they take.
 //   * blocks of query rows: about 1,024 over the launch, but at least two
 //     slots per counted key (the table costs 4 B per key and block)
 //   * segments: about 32,768 over the launch, 256 to 4,096 entries
@@ -951,15 +992,11 @@ GradLayout grad_plan(GradP &p, int det) {
     L.poison = take(keys + 4);
     L.segs = take((int64_t)p.ng * p.segcap * (int64_t)sizeof(GradSeg));
     L.nseg = take((int64_t)p.ng * 4);
+    const bool parts = p.grows < (int64_t)p.a.rep * p.a.N;
+    L.acc = take(parts ? (int64_t)p.a.M * 2 * p.a.d * (det ? 8 : 4) : 0);
     L.part = take((int64_t)p.ng * p.partcap * 2 * p.a.d * (det ? 16 : 4));
     L.total = o;
     return L;
-}
-
-int grad_groups(const GradP &p) {
-    const int64_t all = (int64_t)p.a.B * p.a.Hkv;
-    const int64_t fit = p.gslots > 0 ? GRAD_SLOTS / p.gslots : all;
-    return (int)std::max<int64_t>(1, std::min(all, fit));
 }
 
 // K and V rows within 32-bit byte offsets of a wave-uniform base, rows
@@ -972,14 +1009,13 @@ bool grad_off32(const ApplyP &p, int elem, int D) {
 }
 
 template <typename T, typename TD, int D, int U, bool OFF32>
-int launch_rows(const GradP &p, unsigned grid, hipStream_t st) {
+int launch_rows(const GradP &p, dim3 grid, hipStream_t st) {
     constexpr int STEP = Geo<T, D>::RPI * U;
     const size_t lds = (size_t)WAVES * 3 * ceil_div(p.a.K, STEP) * STEP * 4;
     if (lds > 65536)
         SSA_CHECK_HIP(hipFuncSetAttribute((const void *)grad_rows_kernel<T, TD, D, U, OFF32>,
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((grad_rows_kernel<T, TD, D, U, OFF32>), dim3(grid), dim3(WAVES * SSA_WAVE), lds,
-                       st, p);
+    hipLaunchKernelGGL((grad_rows_kernel<T, TD, D, U, OFF32>), grid, dim3(WAVES * SSA_WAVE), lds, st, p);
     SSA_CHECK_LAUNCH();
     return SSA_OK;
 }
@@ -987,8 +1023,10 @@ int launch_rows(const GradP &p, unsigned grid, hipStream_t st) {
 template <typename T, typename TD, int D>
 int launch_grad(GradP p, int det, char *ws, hipStream_t st) {
     constexpr int U = grad_u<T, D>();
-    const int all = p.a.B * p.a.Hkv, per = grad_groups(p);
-    p.ng = per;
+    const int all = p.a.B * p.a.Hkv;
+    grad_launches(p);
+    const int per = p.ng;
+    const int64_t rows = (int64_t)p.a.rep * p.a.N, part = p.grows;
     const GradLayout L = grad_plan(p, det);
     p.ent = (uint4 *)(ws + L.ent);
     p.rank = (uint32_t *)(ws + L.rank);
@@ -1002,49 +1040,63 @@ int launch_grad(GradP p, int det, char *ws, hipStream_t st) {
     p.poison = (uint8_t *)(ws + L.poison);
     p.segs = (GradSeg *)(ws + L.segs);
     p.nseg = (int32_t *)(ws + L.nseg);
+    p.acc = ws + L.acc;
     p.part = ws + L.part;
     const ApplyP &a = p.a;
     const size_t clds = (size_t)std::min(a.M, CNT_KEYS) * 4;
-    for (int g0 = 0; g0 < all; g0 += per) {
-        p.g0 = g0;
-        p.ng = std::min(per, all - g0);
-        hipLaunchKernelGGL(grad_count_kernel, dim3((unsigned)p.ng * (unsigned)p.nc), dim3(CNT_THREADS),
-                           clds, st, p);
+    // the launches of the groups and rows that p holds
+    auto launch = [&]() -> int {
+        hipLaunchKernelGGL(grad_count_kernel, launch_grid((int64_t)p.ng * p.nc), dim3(CNT_THREADS), clds,
+                           st, p);
         SSA_CHECK_LAUNCH();
         const int64_t keys = (int64_t)p.ng * a.M;
-        hipLaunchKernelGGL(grad_chunk_kernel, dim3((unsigned)ceil_div(keys, 256)), dim3(256), 0, st, p);
+        hipLaunchKernelGGL(grad_chunk_kernel, launch_grid(ceil_div(keys, 256)), dim3(256), 0, st, p);
         SSA_CHECK_LAUNCH();
-        hipLaunchKernelGGL(grad_list_kernel, dim3((unsigned)p.ng), dim3(1024), 0, st, p);
+        hipLaunchKernelGGL(grad_list_kernel, launch_grid(p.ng), dim3(1024), 0, st, p);
         SSA_CHECK_LAUNCH();
-        hipLaunchKernelGGL(grad_segs_kernel, dim3((unsigned)ceil_div(keys, 256)), dim3(256), 0, st, p);
+        hipLaunchKernelGGL(grad_segs_kernel, launch_grid(ceil_div(keys, 256)), dim3(256), 0, st, p);
         SSA_CHECK_LAUNCH();
-        const unsigned grid = (unsigned)(8 * ceil_div(ceil_div((int64_t)p.ng * p.grows, WAVES), 8));
+        const dim3 grid = launch_grid(8 * ceil_div(ceil_div((int64_t)p.ng * p.grows, WAVES), 8));
         if (a.K > GRAD_KLDS) {
-            hipLaunchKernelGGL((grad_rows_long_kernel<T, TD, D>), dim3(grid), dim3(WAVES * SSA_WAVE), 0,
-                               st, p);
+            hipLaunchKernelGGL((grad_rows_long_kernel<T, TD, D>), grid, dim3(WAVES * SSA_WAVE), 0, st, p);
             SSA_CHECK_LAUNCH();
         } else {
             const int rc = grad_off32(a, (int)sizeof(T), D) ? launch_rows<T, TD, D, U, true>(p, grid, st)
                                                             : launch_rows<T, TD, D, U, false>(p, grid, st);
             if (rc) return rc;
         }
-        const unsigned kgrid = (unsigned)(8 * ceil_div(ceil_div(p.segcap, WAVES) * p.ng, 8));
+        const dim3 kgrid = launch_grid(8 * ceil_div(ceil_div(p.segcap, WAVES) * p.ng, 8));
         constexpr int UK = U > 4 ? 4 : U;
-        const unsigned jgrid = (unsigned)ceil_div(keys, WAVES);
+        const dim3 jgrid = launch_grid(ceil_div(keys, WAVES));
         if (det) {
-            hipLaunchKernelGGL(grad_bound_kernel, dim3(kgrid), dim3(WAVES * SSA_WAVE), 0, st, p);
+            hipLaunchKernelGGL(grad_bound_kernel, kgrid, dim3(WAVES * SSA_WAVE), 0, st, p);
             SSA_CHECK_LAUNCH();
-            hipLaunchKernelGGL((grad_keys_kernel<T, TD, D, 2, true>), dim3(kgrid),
-                               dim3(WAVES * SSA_WAVE), 0, st, p);
+            hipLaunchKernelGGL((grad_keys_kernel<T, TD, D, 2, true>), kgrid, dim3(WAVES * SSA_WAVE), 0, st,
+                               p);
             SSA_CHECK_LAUNCH();
-            hipLaunchKernelGGL((grad_join_kernel<T, true>), dim3(jgrid), dim3(WAVES * SSA_WAVE), 0, st, p);
+            hipLaunchKernelGGL((grad_join_kernel<T, true>), jgrid, dim3(WAVES * SSA_WAVE), 0, st, p);
         } else {
-            hipLaunchKernelGGL((grad_keys_kernel<T, TD, D, UK, false>), dim3(kgrid),
-                               dim3(WAVES * SSA_WAVE), 0, st, p);
+            hipLaunchKernelGGL((grad_keys_kernel<T, TD, D, UK, false>), kgrid, dim3(WAVES * SSA_WAVE), 0,
+                               st, p);
             SSA_CHECK_LAUNCH();
-            hipLaunchKernelGGL((grad_join_kernel<T, false>), dim3(jgrid), dim3(WAVES * SSA_WAVE), 0, st, p);
+            hipLaunchKernelGGL((grad_join_kernel<T, false>), jgrid, dim3(WAVES * SSA_WAVE), 0, st, p);
         }
         SSA_CHECK_LAUNCH();
+        return SSA_OK;
+    };
+    for (int g0 = 0; g0 < all; g0 += per) {
+        p.g0 = g0;
+        p.ng = std::min(per, all - g0);
+        for (int64_t r0 = 0; r0 < rows; r0 += part) {
+            p.r0 = r0;
+            p.row0 = g0 * rows + r0;
+            p.grows = std::min(part, rows - r0);
+            p.gslots = p.grows * a.K;
+            p.first = r0 == 0;
+            p.last = r0 + part >= rows;
+            const int rc = launch();
+            if (rc) return rc;
+        }
     }
     return SSA_OK;
 }
@@ -1125,8 +1177,6 @@ int grad_common(const ssa_apply_grad_args *a, GradP &p) {
     p.dk = (void *)a->dk.ptr; p.dksb = a->dk.sb; p.dksh = a->dk.sh; p.dksn = a->dk.sn;
     p.dv = (void *)a->dv.ptr; p.dvsb = a->dv.sb; p.dvsh = a->dv.sh; p.dvsn = a->dv.sn;
     p.out32 = a->dq.dtype == SSA_F32;
-    p.grows = (int64_t)p.a.rep * p.a.N;
-    p.gslots = p.grows * p.a.K;
     // entries hold offsets of q and dO rows from their group's first in 32
     // bits, in the largest unit (up to 8 elements) that divides the strides
     const int64_t all = p.a.qsh | p.a.qsn | p.dosh | p.dosn;
@@ -1142,7 +1192,7 @@ int grad_common(const ssa_apply_grad_args *a, GradP &p) {
 
 int grad_run_checked(GradP &p, const ssa_apply_grad_args *a, void *ws, int64_t wsb, void *stream) {
     GradP q = p;
-    q.ng = grad_groups(q);
+    grad_launches(q);
     const int64_t need = grad_plan(q, a->deterministic).total;
     SSA_CHECK_ARG(ws != nullptr && wsb >= need,
                   "sparse_gather_attention_grad: workspace of %lld bytes, %lld needed", (long long)wsb,
@@ -1175,7 +1225,7 @@ extern "C" int64_t ssa_sparse_gather_attention_grad_workspace_bytes(const ssa_ap
     GradP p;
     const int rc = grad_common(a, p);
     if (rc) return rc;
-    p.ng = grad_groups(p);
+    grad_launches(p);
     return grad_plan(p, a->deterministic).total;
 }
 

@@ -325,3 +325,38 @@ def test_deterministic_sums_keep_their_bits_beside_an_outlier(dtype, size):
     err = ((dv.double() - exp).abs() / absum)[..., keep].max().item()
     print(f"  outlier {size:.0e}: {err:.2e}", flush=True)
     assert err <= BAR[dtype]
+
+
+@pytest.mark.parametrize("dtype,det", [(torch.float32, False), (torch.float32, True),
+                                       (torch.bfloat16, True)])
+def test_gradients_of_a_group_in_parts(dtype, det):
+    """One group of more than 2^28 slots goes in two parts of its query rows:
+    dq equals that of calls on the parts' rows, dk and dv the sum of theirs."""
+    from ssa_amd import _lib
+    N, M, d, K = (1 << 18) + 1000, 64, 8, 1024
+    g = torch.Generator(DEV).manual_seed(9)
+    q, dout = (torch.randn(1, 1, N, d, generator=g, device=DEV).to(dtype) for _ in range(2))
+    k, v = (torch.randn(1, 1, M, d, generator=g, device=DEV).to(dtype) for _ in range(2))
+    nb = torch.randint(0, M - 1, (1, 1, N, K), generator=g, device=DEV, dtype=torch.int32)
+    got = _lib.gather_attention_grad(q, k, v, nb, None, 0.3, False, 0.0, 0, dout, det)
+    if det:
+        again = _lib.gather_attention_grad(q, k, v, nb, None, 0.3, False, 0.0, 0, dout, det)
+        assert all(torch.equal(a, b) for a, b in zip(got, again))
+    parts = [_lib.gather_attention_grad(q[:, :, s], k, v, nb[:, :, s].contiguous(), None, 0.3,
+                                        False, 0.0, 0, dout[:, :, s], True)
+             for s in (slice(0, 100000), slice(100000, N))]
+    assert torch.equal(got[0], torch.cat([p[0] for p in parts], 2))
+    for a, b, c in zip(got[1:], *(p[1:] for p in parts)):
+        exp = b.double() + c.double()
+        assert (a[0, 0, M - 1] == 0).all()
+        rel = ((a.double() - exp).norm() / exp.norm()).item()
+        assert rel <= (2e-6 if dtype == torch.float32 else 4e-3), rel
+
+
+def test_gradients_of_more_key_rows_than_a_launch_takes():
+    """2^26 key rows under two query rows a batch: launches of 2^25 key rows."""
+    from ssa_amd import _lib
+    B, M, d, K = 1024, 65536, 4, 3
+    q, k, v, nb, va, dout = _inputs(B, 1, 1, 2, M, d, K, torch.float32, 29)
+    got = _lib.gather_attention_grad(q, k, v, nb, va, 0.5, False, 0.0, 0, dout, False)
+    _check(got, _reference(q, k, v, nb, va, 0.5, dout), torch.float32)
