@@ -52,7 +52,7 @@ struct GradP {
     int64_t dqsb, dqsh, dqsn, dksb, dksh, dksn, dvsb, dvsh, dvsn;
     int32_t out32;         // gradients are fp32 (else q's type)
     int32_t accumulate;    // dk, dv are added to (fp32 only)
-    int32_t shift;         // entries hold row offsets in units of 1 << shift elements
+    int32_t shift;         // entries hold row offsets in units of 1 << shift elements; -1: rows
     // groups (b, kv head) of this launch: [g0, g0 + ng), with all their query rows,
     // or one group's rows from r0 on (a part: the first, the last, or between)
     int32_t g0, ng;
@@ -64,7 +64,7 @@ struct GradP {
     int32_t seg;           // entries per segment
     int64_t segcap, partcap;
     // workspace
-    uint4 *ent;            // (ng * gslots) {q offset, dO offset, draw, p'}
+    uint4 *ent;            // (ng * gslots) {q offset, dO offset, draw, p'} ({row, -, ..})
     uint32_t *rank;        // (ng * gslots)
     uint32_t *tab;         // (ng, nc, M) slots before this block
     int64_t *kbegin;       // (ng, M)
@@ -359,8 +359,13 @@ struct RowOut {
         tab = p.tab + ((int64_t)gl * p.nc + c) * p.a.M;
         rank = p.rank + lrow * p.a.K;
         slot = row * p.a.K;
-        qoff = (uint32_t)(((int64_t)hl * p.a.qsh + (int64_t)n * p.a.qsn) >> p.shift);
-        dooff = (uint32_t)(((int64_t)hl * p.dosh + (int64_t)n * p.dosn) >> p.shift);
+        if (p.shift >= 0) {
+            qoff = (uint32_t)(((int64_t)hl * p.a.qsh + (int64_t)n * p.a.qsn) >> p.shift);
+            dooff = (uint32_t)(((int64_t)hl * p.dosh + (int64_t)n * p.dosn) >> p.shift);
+        } else {
+            qoff = (uint32_t)(lrow - (int64_t)gl * p.grows);
+            dooff = 0u;
+        }
     }
     __device__ __forceinline__ void put(const GradP &p, int x, int j, float draw, float pw) const {
         if (x >= 0) {
@@ -798,8 +803,17 @@ grad_keys_kernel(GradP gp) {
         bool zero = false;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            qr[u] = load_raw<T, VEC>(qb + ((uint64_t)en[u].x << gp.shift));
-            dr[u] = load_raw<TD, VEC>(db + ((uint64_t)en[u].y << gp.shift));
+            int64_t qo, dO;
+            if (gp.shift >= 0) {
+                qo = (int64_t)((uint64_t)en[u].x << gp.shift);
+                dO = (int64_t)((uint64_t)en[u].y << gp.shift);
+            } else {
+                const int64_t r = gp.r0 + en[u].x, hl = r / p.N, n = r - hl * p.N;
+                qo = hl * p.qsh + n * p.qsn;
+                dO = hl * gp.dosh + n * gp.dosn;
+            }
+            qr[u] = load_raw<T, VEC>(qb + qo);
+            dr[u] = load_raw<TD, VEC>(db + dO);
             const bool in = j0 + u * RPI + sub < sg.len;
             wk[u] = in ? __uint_as_float(en[u].z) : 0.f;
             wv[u] = in ? __uint_as_float(en[u].w) : 0.f;
@@ -1183,10 +1197,9 @@ int grad_common(const ssa_apply_grad_args *a, GradP &p) {
     p.shift = (all & 1) ? 0 : (all & 2) ? 1 : (all & 4) ? 2 : 3;
     auto span = [&](int64_t sh, int64_t sn) { return (p.a.rep - 1) * sh + (int64_t)std::max(p.a.N - 1, 0) * sn; };
     const bool neg = p.a.qsh < 0 || p.a.qsn < 0 || p.dosh < 0 || p.dosn < 0;
-    if (neg || (std::max(span(p.a.qsh, p.a.qsn), span(p.dosh, p.dosn)) >> p.shift) >= ((int64_t)1 << 32)) {
-        ssa_set_error("sparse_gather_attention_grad: query rows of one kv head beyond 32-bit offsets");
-        return SSA_E_UNSUP;
-    }
+    // (rows farther apart, or backwards: the entries hold the rows' numbers)
+    if (neg || (std::max(span(p.a.qsh, p.a.qsn), span(p.dosh, p.dosn)) >> p.shift) >= ((int64_t)1 << 32))
+        p.shift = -1;
     return SSA_OK;
 }
 

@@ -360,3 +360,22 @@ def test_gradients_of_more_key_rows_than_a_launch_takes():
     q, k, v, nb, va, dout = _inputs(B, 1, 1, 2, M, d, K, torch.float32, 29)
     got = _lib.gather_attention_grad(q, k, v, nb, va, 0.5, False, 0.0, 0, dout, False)
     _check(got, _reference(q, k, v, nb, va, 0.5, dout), torch.float32)
+
+
+@pytest.mark.parametrize("det", [False, True])
+@pytest.mark.parametrize("which", ["q", "dout"])
+def test_gradients_of_query_rows_far_apart(which, det):
+    """Two query heads of one kv head 2^32 + 1 elements apart (an odd stride, so
+    no unit fits 32 bits): the gradients of the same rows side by side."""
+    from ssa_amd import _lib
+    q, k, v, nb, va, dout = _inputs(1, 2, 1, 70, 50, 32, 37, torch.bfloat16, 31)
+    base = _lib.gather_attention_grad(q, k, v, nb, va, 0.2, False, 0.0, 0, dout, det)
+    far = torch.empty((1 << 32) + 70 * 33 + 64, dtype=torch.bfloat16, device=DEV).as_strided(
+        (1, 2, 70, 32), (1 << 33, (1 << 32) + 1, 33, 1))
+    far.copy_(q if which == "q" else dout)
+    got = _lib.gather_attention_grad(far if which == "q" else q, k, v, nb, va, 0.2, False, 0.0, 0,
+                                     far if which == "dout" else dout, det)
+    for name, a, b in zip(("dq", "dk", "dv"), got, base):
+        if det or name == "dq":
+            assert torch.equal(a, b), name
+        _check_grad_rows(name, a, b, torch.bfloat16)

@@ -46,3 +46,13 @@ def test_workspace_of_many_key_rows_is_bounded():
     one = _bytes(_args(512, 1, 1, 2, 65536, 8, 3))
     assert one <= (1 << 25) * 62 + (1 << 20)
     assert _bytes(_args(4096, 1, 1, 2, 65536, 8, 3)) <= one + (1 << 20)
+
+
+@pytest.mark.parametrize("det", [False, True])
+def test_any_strides_of_q_and_dout_are_taken(det):
+    """Query rows of a kv head beyond 32-bit offsets from each other, as the
+    forward takes them."""
+    far, back = (1 << 40, (1 << 32) + 1, 17), (1 << 20, -(1 << 10), 16)
+    want = _bytes(_args(1, 2, 1, 4, 8, 16, 3, det=det))
+    for kw in (dict(q=far), dict(dout=far), dict(q=back), dict(dout=back)):
+        assert _bytes(_args(1, 2, 1, 4, 8, 16, 3, det=det, **kw)) == want
