@@ -108,6 +108,21 @@ int64_t ssa_graph_workspace_bytes(const ssa_graph_args *a);
 int ssa_build_graph(const ssa_graph_args *a, void *workspace, int64_t workspace_bytes,
                     void *stream);
 
+/* The build's two forms (no counterpart in the reference): over the lists'
+ * members, or (FULL mode, at most 4,096 keys and 64 lists) over every key.  Both
+ * give the same graph; ssa_build_graph takes the one its rule says is faster.  For
+ * tests and measurements of either: ssa_graph_form returns the form ssa_build_graph
+ * (noalloc: ssa_build_graph_noalloc) takes for these arguments, or a negative code;
+ * the other two are ssa_graph_workspace_bytes and ssa_build_graph in the form
+ * given, SSA_E_UNSUP where it does not take the sizes. */
+#define SSA_FORM_AUTO  0
+#define SSA_FORM_LIST  1
+#define SSA_FORM_DENSE 2
+int ssa_graph_form(const ssa_graph_args *a, int32_t noalloc);
+int64_t ssa_graph_form_workspace_bytes(const ssa_graph_args *a, int32_t form);
+int ssa_build_graph_form(const ssa_graph_args *a, int32_t form, void *workspace,
+                         int64_t workspace_bytes, void *stream);
+
 /* ssa_build_graph without any device allocation (no counterpart in the
  * reference): for callers that cannot allocate -- code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  The same

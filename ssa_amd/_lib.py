@@ -20,6 +20,7 @@ LIB_PATH = os.path.join(_HERE, "libssa_amd.so")
 
 SSA_F32, SSA_BF16, SSA_F16 = 0, 1, 2
 GRAPH_FULL, GRAPH_LSH = 0, 1
+FORM_AUTO, FORM_LIST, FORM_DENSE = 0, 1, 2
 
 _DTYPES = {torch.float32: SSA_F32, torch.bfloat16: SSA_BF16, torch.float16: SSA_F16}
 
@@ -135,6 +136,12 @@ def _configure(L):
     L.ssa_graph_workspace_bytes.argtypes = [ctypes.POINTER(GraphArgs)]
     L.ssa_build_graph.restype = ctypes.c_int
     L.ssa_build_graph.argtypes = [ctypes.POINTER(GraphArgs), c_vp, c_i64, c_vp]
+    L.ssa_graph_form.restype = ctypes.c_int
+    L.ssa_graph_form.argtypes = [ctypes.POINTER(GraphArgs), c_i32]
+    L.ssa_graph_form_workspace_bytes.restype = c_i64
+    L.ssa_graph_form_workspace_bytes.argtypes = [ctypes.POINTER(GraphArgs), c_i32]
+    L.ssa_build_graph_form.restype = ctypes.c_int
+    L.ssa_build_graph_form.argtypes = [ctypes.POINTER(GraphArgs), c_i32, c_vp, c_i64, c_vp]
     L.ssa_build_graph_noalloc.restype = ctypes.c_int
     L.ssa_build_graph_noalloc.argtypes = [ctypes.POINTER(GraphArgs), c_vp]
     L.ssa_project_graph_supported.restype = ctypes.c_int
@@ -284,6 +291,18 @@ def _graph_args(q, k, rand_proj, *, P, T, C, top_k, window, causal, is_cross, to
     return a, [qk, kk_, rp, g, qp, kp]
 
 
+def graph_form(q, k, rand_proj, *, noalloc=False, **kw) -> int:
+    """The form (FORM_LIST or FORM_DENSE) build_graph takes for these arguments
+    (ssa_graph_form)."""
+    dp = kernel_head_dim(q.shape[-1], q.dtype)
+    a, _ = _graph_args(_pad_cols(q, dp), _pad_cols(k, dp), _pad_cols(rand_proj, dp),
+                       q_proj=None, k_proj=None, **{"mode": GRAPH_FULL, **kw})
+    rc = lib().ssa_graph_form(ctypes.byref(a), int(noalloc))
+    if rc < 0:
+        _check(rc, "graph_form")
+    return rc
+
+
 def _graph_outputs(a, width, mode, ids32, count_ties, device):
     """Allocate the graph outputs for width slots and point `a` at them."""
     B, Hq, N = a.B, a.Hq, a.N
@@ -324,15 +343,16 @@ def _pad_cols(t, dp):
 
 def build_graph(q, k, rand_proj, *, P, T, C, top_k, window, causal, is_cross, total_k, glob,
                 mode=GRAPH_FULL, q_proj=None, k_proj=None, count_ties=False, ids32=False,
-                noalloc=False):
+                noalloc=False, form=FORM_AUTO):
     """Run ssa_build_graph.  q (B,Hq,N,d), k (B,Hkv,M,d) views on one device.
 
     Returns (out_idx, out_valid or None, ties or None).  With ids32 (FULL mode)
     out_idx is int32 with -1 in the invalid slots and out_valid is None.  With
     noalloc the build runs through ssa_build_graph_noalloc: no workspace is
     allocated (the library's fixed scratch array serves instead; the outputs
-    are still allocated here).  Head dims the kernels do not take run
-    zero-padded (kernel_head_dim)."""
+    are still allocated here).  form: FORM_LIST or FORM_DENSE instead of the
+    library's choice (ssa_build_graph_form; the graph is the same).  Head dims
+    the kernels do not take run zero-padded (kernel_head_dim)."""
     if q.dim() == 4 and k.dim() == 4 and q.shape[-1] == k.shape[-1]:
         dp = kernel_head_dim(q.shape[-1], q.dtype)
         q, k = _pad_cols(q, dp), _pad_cols(k, dp)
@@ -345,7 +365,10 @@ def build_graph(q, k, rand_proj, *, P, T, C, top_k, window, causal, is_cross, to
     width = L.ssa_graph_out_width(ctypes.byref(a))
     if width < 0:
         _check(-1, "build_graph")
-    wsb = 0 if noalloc else L.ssa_graph_workspace_bytes(ctypes.byref(a))
+    if form and noalloc:
+        raise RuntimeError("ssa_amd.build_graph: noalloc takes no form")
+    wsb = 0 if noalloc else (L.ssa_graph_form_workspace_bytes(ctypes.byref(a), form) if form
+                             else L.ssa_graph_workspace_bytes(ctypes.byref(a)))
     if wsb < 0:
         _check(-1, "build_graph")
     out, valid, ties = _graph_outputs(a, width, mode, ids32, count_ties, q.device)
@@ -355,8 +378,11 @@ def build_graph(q, k, rand_proj, *, P, T, C, top_k, window, causal, is_cross, to
             _check(L.ssa_build_graph_noalloc(ctypes.byref(a), _stream(q)), "build_graph_noalloc")
     else:
         ws = torch.empty(max(int(wsb), 1), dtype=torch.uint8, device=q.device)
-        _check(L.ssa_build_graph(ctypes.byref(a), ws.data_ptr(), int(wsb), _stream(q)),
-               "build_graph")
+        if form:
+            rc = L.ssa_build_graph_form(ctypes.byref(a), form, ws.data_ptr(), int(wsb), _stream(q))
+        else:
+            rc = L.ssa_build_graph(ctypes.byref(a), ws.data_ptr(), int(wsb), _stream(q))
+        _check(rc, "build_graph")
     # keep inputs alive until the stream has consumed them
     keep.append(ws)
     del keep

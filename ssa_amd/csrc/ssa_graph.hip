@@ -3611,9 +3611,14 @@ Layout plan(const Dims &D) {
     return L;
 }
 
-// Whether the build takes the dense form (ssa_graph_dense.h): a graph, keys
-// within a select row's registers, lists within a wave's lanes, a round's
-// bitmaps within LDS, and enough list members (over a row's lists) per key.
+// What the dense form (ssa_graph_dense.h) takes: a graph, keys within a select
+// row's registers, lists within a wave's lanes, a round's bitmaps within LDS.
+bool dense_fits(const Dims &D, const ssa_graph_args *a) {
+    return a->mode == SSA_GRAPH_FULL && D.M <= DN_MAX_KEYS && D.nlists <= DN_MAX_LISTS &&
+           D.NB * (ceil_div(D.M, 64) * 8 + 4) <= DN_BITS_LDS;
+}
+
+// Whether the build takes it: enough list members (over a row's lists) per key.
 // Where that line lies was measured with both forms (whole build, list / dense
 // us): 16-bit rows, 4,096 causal keys, d = 64: 0.9 members per key 413 / 436,
 // 1.8: 753 / 621; 2,048 keys: 0.8: 188 / 187, 1.8: 234 / 191; 1,024 keys: 0.25:
@@ -3622,10 +3627,7 @@ Layout plan(const Dims &D) {
 // 602 (causal), 0.4: 535 / 550 and 836 / 731; 2,048 keys: 0.4: 352 / 322 and 324 /
 // 251; 1,024 keys: 0.25: 293 / 200.
 bool dense_form(const Dims &D, const ssa_graph_args *a) {
-    const int64_t nw = ceil_div(D.M, 64);
-    if (a->mode != SSA_GRAPH_FULL || D.M > DN_MAX_KEYS || D.nlists > DN_MAX_LISTS ||
-        D.NB * (nw * 8 + 4) > DN_BITS_LDS)
-        return false;
+    if (!dense_fits(D, a)) return false;
     const int64_t members = (int64_t)D.nlists * std::min<int64_t>(D.C, ceil_div(D.M, D.NB));
     if (D.M <= 1024) return members * 4 >= D.M;
     return a->q.dtype == SSA_F32 ? members * 5 >= (int64_t)D.M * 2 : members >= D.M;
@@ -3635,9 +3637,10 @@ Layout plan(const Dims &D);
 
 // ws_cap > 0: query heads go in chunks small enough that the workspace stays
 // within ws_cap bytes (the build without allocation runs in a fixed scratch
-// array); SSA_E_WORKSPACE when even one head per chunk needs more.
+// array); SSA_E_WORKSPACE when even one head per chunk needs more.  form:
+// SSA_FORM_LIST / _DENSE in place of the rule's choice.
 int make_dims(const ssa_graph_args *a, Dims &D, bool need_q = true, int64_t ws_cap = 0,
-              bool fused = false) {
+              bool fused = false, int form = SSA_FORM_AUTO) {
     SSA_CHECK_ARG(a != nullptr, "build_graph: null args");
     SSA_CHECK_ARG(a->mode == SSA_GRAPH_FULL || a->mode == SSA_GRAPH_LSH, "build_graph: bad mode");
     SSA_CHECK_ARG(a->B >= 1 && a->Hq >= 1 && a->Hkv >= 1 && a->N >= 1 && a->M >= 1,
@@ -3779,7 +3782,12 @@ int make_dims(const ssa_graph_args *a, Dims &D, bool need_q = true, int64_t ws_c
         const int64_t per = D.dense ? (int64_t)D.N * D.Ms * 2 : per_bh;
         D.nbh_chunk = (int)std::max<int64_t>(1, std::min(((int64_t)8 << 30) / per, D.BH));
     };
-    D.dense = dense_form(D, a) ? 1 : 0;
+    if (form == SSA_FORM_DENSE && !dense_fits(D, a)) {
+        ssa_set_error("build_graph: the dense form takes graphs of up to %d keys and %d lists, with a "
+                      "round's bitmaps in %d bytes", DN_MAX_KEYS, DN_MAX_LISTS, DN_BITS_LDS);
+        return SSA_E_UNSUP;
+    }
+    D.dense = form == SSA_FORM_AUTO ? dense_form(D, a) : form == SSA_FORM_DENSE;
     chunk_heads();
     if (ws_cap > 0 && D.dense) {
         // the list form where the dense one does not fit with one head per chunk
@@ -4681,9 +4689,9 @@ extern "C" int64_t ssa_graph_workspace_bytes(const ssa_graph_args *a) {
 
 namespace {
 int build_impl(const ssa_graph_args *a, void *workspace, int64_t workspace_bytes, void *stream,
-               int64_t ws_cap = 0) {
+               int64_t ws_cap = 0, int form = SSA_FORM_AUTO) {
     Dims D;
-    int rc = make_dims(a, D, true, ws_cap);
+    int rc = make_dims(a, D, true, ws_cap, false, form);
     if (rc) return rc;
     {
         const bool i32 = a->mode == SSA_GRAPH_FULL && a->out_idx32;
@@ -4726,6 +4734,27 @@ int build_impl(const ssa_graph_args *a, void *workspace, int64_t workspace_bytes
 extern "C" int ssa_build_graph(const ssa_graph_args *a, void *workspace, int64_t workspace_bytes,
                                void *stream) {
     return build_impl(a, workspace, workspace_bytes, stream);
+}
+
+extern "C" int ssa_graph_form(const ssa_graph_args *a, int32_t noalloc) {
+    Dims D;
+    const int rc = make_dims(a, D, false, noalloc ? (int64_t)SSA_NOALLOC_SCRATCH_BYTES : 0);
+    if (rc) return rc;
+    return D.dense ? SSA_FORM_DENSE : SSA_FORM_LIST;
+}
+
+extern "C" int64_t ssa_graph_form_workspace_bytes(const ssa_graph_args *a, int32_t form) {
+    SSA_CHECK_ARG(form >= SSA_FORM_AUTO && form <= SSA_FORM_DENSE, "build_graph: form %d", form);
+    Dims D;
+    const int rc = make_dims(a, D, false, 0, false, form);
+    if (rc) return rc;
+    return plan(D).total;
+}
+
+extern "C" int ssa_build_graph_form(const ssa_graph_args *a, int32_t form, void *workspace,
+                                    int64_t workspace_bytes, void *stream) {
+    SSA_CHECK_ARG(form >= SSA_FORM_AUTO && form <= SSA_FORM_DENSE, "build_graph: form %d", form);
+    return build_impl(a, workspace, workspace_bytes, stream, 0, form);
 }
 
 int64_t ssa_graph_workspace_bytes_capped(const ssa_graph_args *a, int64_t ws_cap) {

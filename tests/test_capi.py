@@ -66,6 +66,7 @@ def test_struct_layouts_match_the_header(tmp_path):
         pytest.skip("no C compiler")
     mirrors = {"ssa_tensor4": _lib.Tensor4, "ssa_graph_args": _lib.GraphArgs,
                "ssa_apply_args": _lib.ApplyArgs, "ssa_apply_bwd_args": _lib.ApplyBwdArgs,
+               "ssa_apply_grad_args": _lib.ApplyGradArgs,
                "ssa_project_graph_args": _lib.ProjectGraphArgs}
     lines = ['#include <stdio.h>', '#include <stddef.h>', '#include "ssa_amd.h"', 'int main(void) {']
     for cname, py in mirrors.items():

@@ -66,7 +66,7 @@ SIZES = [(1, 2, 1, 63, 63, 16, 2, 3, 0, 40, 2, 1, True, False),
          (1, 1, 1, 4096, 4096, 16, 16, 4, 0, 128, 16, 2, True, False),
          (1, 1, 1, 30, 4097, 16, 16, 4, 0, 128, 2, 2, False, True),
          (1, 1, 1, 100, 100, 16, 64, 3, 0, 40, 2, 2, True, False),
-         (1, 1, 1, 100, 100, 16, 13, 4, 4, 40, 2, 2, True, False)]
+         (1, 1, 1, 100, 100, 16, 65, 3, 0, 40, 2, 2, True, False)]
 
 
 @pytest.mark.parametrize("case", SIZES, ids=lambda c: f"N{c[3]}_M{c[4]}_d{c[5]}_R{c[6]}_T{c[8]}")
