@@ -22,8 +22,10 @@
 //   5. grad_join_kernel    key rows of several segments: sum of their partials
 //                          (21 us)
 //
-// Numerics: scores, softmax, weights and sums in fp32 as in the forward (16-bit
-// products are exact in fp32).  Deterministic mode: the order of a list's
+// Numerics: scores, dO.V, softmax, weights and sums in fp32 (16-bit products are
+// exact in fp32).  Scores, and dO.V where dout has q's type, are 16-bit rows' pairs
+// by v_dot2, as in the forward; dO.V with an fp32 dout, fp32 rows and rows beyond
+// LDS are chains of fp32 FMAs.  Deterministic mode: the order of a list's
 // entries varies between runs, so its sums are made independent of the order:
 // each term (exact in fp64) is rounded to a grid of its key row coarse enough
 // that every partial sum is exact in fp64, and what the rounding left to a

@@ -4407,8 +4407,9 @@ int keys_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws
     bool done = false;
     SortTopArgs sa{};
     if (D.dense && !D.fused) {
-        // (fused: the queries are not projected yet.)  The sort's top levels; then the segments beside the first head chunk's
-        // scores, which need the aux pass's code scales on the matrix cores
+        // The sort's top levels; then the segments beside the first head chunk's
+        // scores, which need the aux pass's code scales on the matrix cores.
+        // (fused: the queries are not projected yet)
         const int nbh = (int)std::min<int64_t>(D.BH, D.nbh_chunk);
         const bool mfma = rescore_uses_mfma<T>(D.d, rescore_common(D, a, L, ws));
         rc = ssa_sort_top_setup((const uint16_t *)(ws + L.kid), (int)(D.BK * D.R), D.M, D.P,
@@ -4435,8 +4436,7 @@ int keys_typed(const Dims &D, const ssa_graph_args *a, const Layout &L, char *ws
         rc = launch_dense<T>(D, a, L, ws, 0, nbh, mfma, &sa, st);
         if (rc) return rc;
         done = true;
-    } else
-    if constexpr (!std::is_same<T, float>::value) {
+    } else if constexpr (!std::is_same<T, float>::value) {
         if (sort_aux) {
             rc = launch_sort_aux<T>(D, a, L, ws, st);
             done = true;

@@ -145,8 +145,8 @@ __device__ __forceinline__ void dense_mfma_tile(const DnP &p, int64_t phys) {
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
             const int e0 = 32 * s + 8 * lg;
-            qf[i][s] = e0 < p.d ? __builtin_bit_cast(V, *reinterpret_cast<const uint4 *>(qbase + (int64_t)n * p.qsn + e0))
-                                : zero;
+            const T *qe = qbase + (int64_t)n * p.qsn + e0;
+            qf[i][s] = e0 < p.d ? __builtin_bit_cast(V, *reinterpret_cast<const uint4 *>(qe)) : zero;
         }
     }
     // A rows of the pair of tiles at key x: keys x + li and x + 64 + li

@@ -696,8 +696,8 @@ def test_apply_backward_at_bench_head_shape(dtype, fp32w):
                                            (torch.bfloat16, 0.2)])
 def test_deterministic_backward_same_bits_and_matches_autograd(dtype, dropout):
     """Under torch.use_deterministic_algorithms(True) the backward takes
-    ssa_sparse_gather_attention_bwd_det: dK / dV summed as fixed-point
-    integers per key row, so three runs give the same bits; every row of
+    ssa_sparse_gather_attention_grad's deterministic form: dK / dV summed in
+    fp64 on grids of their key row, so three runs give the same bits; every row of
     dq / dk / dv matches float64 autograd (with the dropout mask read off the
     output, as in the dropout test) to the per-row bar.  GQA (8 query heads
     over 2 kv heads), N=M=2048, K=128, d=128, every key reached by several
@@ -731,7 +731,7 @@ def test_deterministic_backward_same_bits_and_matches_autograd(dtype, dropout):
     for gr in grads[1:]:
         for a, b_ in zip(gr, grads[0]):
             assert torch.equal(a, b_)
-    # with dropout the reference is the fp32-atomic backward of the same seed
+    # with dropout the reference is the default backward of the same seed
     # (itself checked against float64 autograd by the dropout test); without,
     # float64 autograd
     if dropout > 0:
