@@ -4318,11 +4318,14 @@ int launch_dense(const Dims &D, const ssa_graph_args *a, const Layout &L, char *
     int nseg = 0;
     size_t lds = mfma ? 0 : DV_LDS;
     const int64_t tiles = (int64_t)dp.qtiles * dp.ktiles * nbh;
-    // A shared launch pays where the tiles outlast the segments or all fit the
-    // chip at once; few long tiles would wait for the slots of the segments'
-    // workgroups, which take the tiles' registers (512 tiles behind 384
-    // segment workgroups: 107 us against 24 + 45 apart).
-    const bool share = segs && (tiles >= 1024 || tiles + ssa_sort_seg_blocks(segs->rows, segs->n) <= 256);
+    // The tiles share the segments' launch, whose workgroups come first and stay,
+    // unless there are several of those a CU and the tiles are the wide ones, whose
+    // registers leave few slots beside them.  Whole builds, bf16, d = 64, in launches
+    // apart / shared, us: narrow tiles beside 512 segment workgroups (16 heads of 2,048)
+    // 198 / 182; wide tiles beside 187 (16 heads of 2,999 on 4 kv heads) 433 / 423, 256:
+    // 847 / 838, 375: 450 / 453, 512: 347 / 360, 750: 406 / 439, 1,024: 299 / 337, 2,048:
+    // 1,087 / 1,239.  fp32 tiles: 0 to 23% less when shared, beside 16 to 2,048.
+    const bool share = segs && (!mfma || !wide || ssa_sort_seg_blocks(segs->rows, segs->n) <= 256);
     if (segs && !share) {
         const int rc = ssa_launch_sort_seg(*segs, st);
         if (rc) return rc;
