@@ -3620,17 +3620,21 @@ bool dense_fits(const Dims &D, const ssa_graph_args *a) {
 
 // Whether the build takes it: enough list members (over a row's lists) per key.
 // Where that line lies was measured with both forms (whole build, list / dense
-// us): 16-bit rows, 4,096 causal keys, d = 64: 0.9 members per key 413 / 436,
+// us): rows the matrix cores take, 4,096 causal keys, d = 64: 0.9 members per key 413 / 436,
 // 1.8: 753 / 621; 2,048 keys: 0.8: 188 / 187, 1.8: 234 / 191; 1,024 keys: 0.25:
-// 177 / 164, 0.8: 156 / 136; 512 keys (cross): 0.5: 223 / 187.  fp32, whose list
-// rescore runs on the vector units: 4,096 keys: 0.2: 384 / 553 (cross) and 520 /
-// 602 (causal), 0.4: 535 / 550 and 836 / 731; 2,048 keys: 0.4: 352 / 322 and 324 /
-// 251; 1,024 keys: 0.25: 293 / 200.
+// 177 / 164, 0.8: 156 / 136; 512 keys (cross): 0.5: 223 / 187.  Rows whose list
+// rescore runs on the vector units, fp32: 4,096 keys: 0.2: 384 / 553 (cross) and
+// 520 / 602 (causal), 0.4: 535 / 550 and 836 / 731; 2,048 keys: 0.4: 352 / 322 and
+// 324 / 251; 1,024 keys: 0.25: 293 / 200; bf16 of d = 160 and 256: 4,096 causal keys:
+// 0.84: 3,203 / 567 and 8,328 / 1,789; 2,048: 0.5: 984 / 230 and 2,231 / 470.
+// (16-bit rows of up to 128 that are not 16-byte aligned stay on the first line: the
+// form may not hang on pointers a size query does not have.)
 bool dense_form(const Dims &D, const ssa_graph_args *a) {
     if (!dense_fits(D, a)) return false;
     const int64_t members = (int64_t)D.nlists * std::min<int64_t>(D.C, ceil_div(D.M, D.NB));
     if (D.M <= 1024) return members * 4 >= D.M;
-    return a->q.dtype == SSA_F32 ? members * 5 >= (int64_t)D.M * 2 : members >= D.M;
+    const bool vector = a->q.dtype == SSA_F32 || D.d < 8 || D.d > 128;
+    return vector ? members * 5 >= (int64_t)D.M * 2 : members >= D.M;
 }
 
 Layout plan(const Dims &D);
