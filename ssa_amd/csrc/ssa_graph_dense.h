@@ -100,7 +100,9 @@ __global__ void __launch_bounds__(1024) list_bits_kernel(LbP p) {
 // ---------------------------------------------------------------- scores
 // 16-query operands per wave (QF): 4, or 2 where 4 leaves fewer than DM_TILES
 // workgroups (64 x 2,048 queries over 512 keys, d = 64: 512 workgroups 69 us,
-// 1,024 of half the queries 50 us)
+// 1,024 of half the queries 50 us).  Whole builds about the line, 4 / 2 operands:
+// 512 workgroups of four 192 / 183 us (16 heads of 2,048, d = 64), 230 / 231 and 269 /
+// 289 (64 heads of 1,024, d = 64 and 128); 1,024: 282 / 277 (32 heads of 2,048, d = 64)
 constexpr int DM_QF = 4, DM_TILES = 1024;
 constexpr int DM_K = 512;              // keys per workgroup: 4 blocks
 
